@@ -10,345 +10,42 @@
 // templates for 4 keys as 4 16-byte loads (the reference pairs its templates likewise,
 // model/attention_cuda.py:410-440).
 //
-// A workgroup takes a run of groups_per_block (position, key/value group) pairs, in order, which may run on
-// from one position into the next; it has one wavefront per slab of 16 queries, or (SPLIT, five slabs in large
-// launches) four wavefronts, three of which share the fifth slab by 32-key step (its queries normalised once in LDS,
-// its parts merged by the fourth while the next group's keys are normalised). A group's raw key, value and
-// query rows arrive by DMA into LDS, double-buffered: the next group's rows load while this group's heads run.
-// The keys are normalised in place in LDS (four threads a key), the queries in registers; a wavefront then runs
-// each head of the group on v_mfma_f32_16x16x32_f16: the scores come out transposed, S^T = K' Q'^T, so a lane
-// holds one query's scores for 4 keys of each 16-key tile -- exactly the fragment O^T = V^T P^T needs as its B
-// operand, so the probabilities never leave registers. V^T's fragments are read from the raw value rows by transposing LDS reads (ds_read_b64_tr_b16: in
-// each 16 lanes, lane j receives element j % 4 of the 8 bytes lanes j / 4 + 4 r address, r = 0..3), so the
-// values are never transposed in LDS. The template bias is an MFMA too, from the templates held in registers.
+// Two kernels: attention_wave.h's, for query and value widths up to 64 and up to 80 tokens (every network's), and this file's,
+// for wider heads and more tokens. Here a workgroup takes a run of groups_per_block (position, key/value group) pairs, in
+// order, which may run on from one position into the next; it has one wavefront per slab of 16 queries. A group's raw key,
+// value and query rows arrive by DMA into LDS, double-buffered: the next group's rows load while this group's heads run. The
+// keys are normalised in place in LDS (four threads a key), the queries in registers; a wavefront then runs each head of
+// the group on v_mfma_f32_16x16x32_f16: the scores come out transposed, S^T = K' Q'^T, so a lane holds one query's scores for
+// 4 keys of each 16-key tile -- exactly the fragment O^T = V^T P^T needs as its B operand, so the probabilities never leave
+// registers. V^T's fragments are read from the raw value rows by transposing LDS reads (ds_read_b64_tr_b16: in each 16
+// lanes, lane j receives element j % 4 of the 8 bytes lanes j / 4 + 4 r address, r = 0..3), so the values are never
+// transposed in LDS. The template bias is an MFMA too, from the templates held in registers.
 // Attention is held to a tolerance, not to bits: its f32 sums run in the MFMA's and the lanes' order (sums of
 // squares are v_dot2_f32_f16 of the fp16 pairs), the norms take IEEE divides and square roots, and the softmax's
 // exponent is one fma into the hardware exp2.
-#include "chess_common.h"
-
-#include <type_traits>
+#include "attention_wave.h"
 
 namespace {
 
-constexpr int MAX_TEMPLATES = 8;
-constexpr long SPLIT_PAIRS = 1024;   // (position, key/value group) pairs from which a 65-80 token launch takes the split slab
-constexpr float LOG2E = 1.44269504f;
-
-typedef __fp16 h2 __attribute__((ext_vector_type(2)));
-#define LDS_SPACE __attribute__((address_space(3)))
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-
-DEVICE float dot2(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, a), __builtin_bit_cast(h2, b), c, false);
-}
-
-// A 16-byte LDS read of DMA'd data as an instruction of its own, waited for by lgkmcnt and passed through an empty
-// asm so that no use moves above the wait: read through a pointer, the compiler would first wait for every DMA in
-// flight (the next group's rows too), unable to tell the addresses apart.
-DEVICE uint4 lds_read16_settled(const LDS_SPACE void* p) {
-    v4u v;
-    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"((uint32_t)(uintptr_t)p) : "memory");
-    return uint4{v[0], v[1], v[2], v[3]};
-}
-
-// The transposing reads of a P V step, for N = DV / 16 column groups: at base[dt] + LO and (HI) base[dt] + HI_OFF, and the
-// wait for them, in one asm statement, so that the values exist only once they have landed. (Read by statements of their
-// own and waited for by another, their registers could be copied by the compiler before the wait, the copy holding what
-// the register held before the read landed.) Without HI the upper half is zero: keys past the staged rows, whose P is zero.
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-template <int N, bool HI> struct StepReads;
-
-template <> struct StepReads<1, true> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[1], v2u (&lo)[1], v2u (&hi)[1]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\t"
-                 "ds_read_b64_tr_b16 %1, %2 offset:%4\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0])
-                 : "v"(base[0]), "i"(LO), "i"(HI_OFF) : "memory");
-    }
-};
-
-template <> struct StepReads<1, false> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[1], v2u (&lo)[1], v2u (&hi)[1]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0])
-                 : "v"(base[0]), "i"(LO) : "memory");
-#pragma unroll
-    for (int dt = 0; dt < 1; dt++) hi[dt] = v2u{0, 0};
-    }
-};
-
-template <> struct StepReads<2, true> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[2], v2u (&lo)[2], v2u (&hi)[2]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%6\n\t"
-                 "ds_read_b64_tr_b16 %1, %4 offset:%7\n\t"
-                 "ds_read_b64_tr_b16 %2, %5 offset:%6\n\t"
-                 "ds_read_b64_tr_b16 %3, %5 offset:%7\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1])
-                 : "v"(base[0]), "v"(base[1]), "i"(LO), "i"(HI_OFF) : "memory");
-    }
-};
-
-template <> struct StepReads<2, false> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[2], v2u (&lo)[2], v2u (&hi)[2]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%4\n\t"
-                 "ds_read_b64_tr_b16 %1, %3 offset:%4\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(lo[1])
-                 : "v"(base[0]), "v"(base[1]), "i"(LO) : "memory");
-#pragma unroll
-    for (int dt = 0; dt < 2; dt++) hi[dt] = v2u{0, 0};
-    }
-};
-
-template <> struct StepReads<4, true> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[4], v2u (&lo)[4], v2u (&hi)[4]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %8 offset:%12\n\t"
-                 "ds_read_b64_tr_b16 %1, %8 offset:%13\n\t"
-                 "ds_read_b64_tr_b16 %2, %9 offset:%12\n\t"
-                 "ds_read_b64_tr_b16 %3, %9 offset:%13\n\t"
-                 "ds_read_b64_tr_b16 %4, %10 offset:%12\n\t"
-                 "ds_read_b64_tr_b16 %5, %10 offset:%13\n\t"
-                 "ds_read_b64_tr_b16 %6, %11 offset:%12\n\t"
-                 "ds_read_b64_tr_b16 %7, %11 offset:%13\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3])
-                 : "v"(base[0]), "v"(base[1]), "v"(base[2]), "v"(base[3]), "i"(LO), "i"(HI_OFF) : "memory");
-    }
-};
-
-template <> struct StepReads<4, false> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[4], v2u (&lo)[4], v2u (&hi)[4]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%8\n\t"
-                 "ds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
-                 "ds_read_b64_tr_b16 %2, %6 offset:%8\n\t"
-                 "ds_read_b64_tr_b16 %3, %7 offset:%8\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3])
-                 : "v"(base[0]), "v"(base[1]), "v"(base[2]), "v"(base[3]), "i"(LO) : "memory");
-#pragma unroll
-    for (int dt = 0; dt < 4; dt++) hi[dt] = v2u{0, 0};
-    }
-};
-
-template <> struct StepReads<8, true> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[8], v2u (&lo)[8], v2u (&hi)[8]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %16 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %1, %16 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %2, %17 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %3, %17 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %4, %18 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %5, %18 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %6, %19 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %7, %19 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %8, %20 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %9, %20 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %10, %21 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %11, %21 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %12, %22 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %13, %22 offset:%25\n\t"
-                 "ds_read_b64_tr_b16 %14, %23 offset:%24\n\t"
-                 "ds_read_b64_tr_b16 %15, %23 offset:%25\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3]), "=&v"(lo[4]), "=&v"(hi[4]), "=&v"(lo[5]), "=&v"(hi[5]), "=&v"(lo[6]), "=&v"(hi[6]), "=&v"(lo[7]), "=&v"(hi[7])
-                 : "v"(base[0]), "v"(base[1]), "v"(base[2]), "v"(base[3]), "v"(base[4]), "v"(base[5]), "v"(base[6]), "v"(base[7]), "i"(LO), "i"(HI_OFF) : "memory");
-    }
-};
-
-template <> struct StepReads<8, false> {
-    template <int LO, int HI_OFF> static DEVICE void read(const uint32_t (&base)[8], v2u (&lo)[8], v2u (&hi)[8]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %8 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %1, %9 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %2, %10 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %3, %11 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %4, %12 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %5, %13 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %6, %14 offset:%16\n\t"
-                 "ds_read_b64_tr_b16 %7, %15 offset:%16\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3]), "=&v"(lo[4]), "=&v"(lo[5]), "=&v"(lo[6]), "=&v"(lo[7])
-                 : "v"(base[0]), "v"(base[1]), "v"(base[2]), "v"(base[3]), "v"(base[4]), "v"(base[5]), "v"(base[6]), "v"(base[7]), "i"(LO) : "memory");
-#pragma unroll
-    for (int dt = 0; dt < 8; dt++) hi[dt] = v2u{0, 0};
-    }
-};
-
-// The split slab's part reads: at lo_base[dt] and hi_base[dt] (immediate offset 0), and their wait, in one asm statement.
-template <int N> DEVICE void part_reads(const uint32_t (&lo_base)[N], const uint32_t (&hi_base)[N], v2u (&lo)[N], v2u (&hi)[N]);
-
-template <> DEVICE void part_reads<1>(const uint32_t (&lo_base)[1], const uint32_t (&hi_base)[1], v2u (&lo)[1], v2u (&hi)[1]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %2\n\t"
-                 "ds_read_b64_tr_b16 %1, %3\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0])
-                 : "v"(lo_base[0]), "v"(hi_base[0]) : "memory");
-}
-
-template <> DEVICE void part_reads<2>(const uint32_t (&lo_base)[2], const uint32_t (&hi_base)[2], v2u (&lo)[2], v2u (&hi)[2]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %4\n\t"
-                 "ds_read_b64_tr_b16 %1, %6\n\t"
-                 "ds_read_b64_tr_b16 %2, %5\n\t"
-                 "ds_read_b64_tr_b16 %3, %7\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1])
-                 : "v"(lo_base[0]), "v"(lo_base[1]), "v"(hi_base[0]), "v"(hi_base[1]) : "memory");
-}
-
-template <> DEVICE void part_reads<4>(const uint32_t (&lo_base)[4], const uint32_t (&hi_base)[4], v2u (&lo)[4], v2u (&hi)[4]) {
-    asm volatile("ds_read_b64_tr_b16 %0, %8\n\t"
-                 "ds_read_b64_tr_b16 %1, %12\n\t"
-                 "ds_read_b64_tr_b16 %2, %9\n\t"
-                 "ds_read_b64_tr_b16 %3, %13\n\t"
-                 "ds_read_b64_tr_b16 %4, %10\n\t"
-                 "ds_read_b64_tr_b16 %5, %14\n\t"
-                 "ds_read_b64_tr_b16 %6, %11\n\t"
-                 "ds_read_b64_tr_b16 %7, %15\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3])
-                 : "v"(lo_base[0]), "v"(lo_base[1]), "v"(lo_base[2]), "v"(lo_base[3]), "v"(hi_base[0]), "v"(hi_base[1]), "v"(hi_base[2]), "v"(hi_base[3]) : "memory");
-}
-
-// f(std::integral_constant<int, I>()) for I = FIRST .. LAST - 1, in order: a loop whose index is a compile-time constant
-template <int FIRST, int LAST, typename F> DEVICE void each_step(F&& f) {
-    if constexpr (FIRST < LAST) {
-        f(std::integral_constant<int, FIRST>());
-        each_step<FIRST + 1, LAST>(f);
-    }
-}
-
-DEVICE void lds_write8(LDS_SPACE void* p, uint2 v) {
-    asm volatile("ds_write_b64 %0, %1" : : "v"((uint32_t)(uintptr_t)p), "v"(v) : "memory");
-}
-
-// The rows in and out are fp16, or bf16 (BF16): raw 16-bit values, widened to f32 where they are used. The normalised
-// queries and keys, the template bias and the QK products stay fp16 either way (normalised values are of order one);
-// with bf16 rows P V runs on the bf16 MFMA, P as a bf16 high part and low part (Probabilities), and the outputs round to
-// bf16.
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-template <bool BF16> DEVICE float widen16(uint32_t bits) {
-    if constexpr (BF16) return __uint_as_float(bits << 16);
-    else return (float)__builtin_bit_cast(half_t, (uint16_t)bits);
-}
-template <bool BF16> DEVICE uint32_t narrow16(float v) {
-    if constexpr (BF16) return __builtin_bit_cast(uint16_t, (__bf16)v);
-    else return __builtin_bit_cast(uint16_t, (half_t)v);
-}
-// two f32 values rounded to 16 bits, a in the low half: the empty asm keeps them f32 values first, so that a product
-// feeding one is not fused into a mixed-precision multiply-and-round (v_fma_mixlo_f16 rounds the exact product once,
-// not the f32 product); the pair converts in one packed instruction
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-template <bool BF16> DEVICE uint32_t narrow16x2(float a, float b) {
-    asm volatile("" : "+v"(a), "+v"(b));
-    if constexpr (BF16) return __builtin_bit_cast(uint32_t, bf2{(__bf16)a, (__bf16)b});
-    else return __builtin_bit_cast(uint32_t, h2{(half_t)a, (half_t)b});
-}
-// a 16-byte chunk of LDS as raw 16-bit values
-DEVICE uint4 lds_chunk(const LDS_SPACE int8_t* p) {
-    const v4u w = *reinterpret_cast<const LDS_SPACE v4u*>(p);
-    return uint4{w[0], w[1], w[2], w[3]};
-}
-
-// 8 raw values (a 16-byte chunk) as f32
-template <bool BF16> DEVICE void widen8(const uint4& w, float (&out)[8]) {
-    const uint32_t words[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        out[2 * i] = widen16<BF16>(words[i] & 0xFFFFu);
-        out[2 * i + 1] = widen16<BF16>(words[i] >> 16);
-    }
-}
-// 8 bf16 values as fp16 (template coefficients of order one)
-DEVICE uint4 bf16_to_f16x8(const uint4& w) {
-    const uint32_t words[4] = {w.x, w.y, w.z, w.w};
-    uint32_t out[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        out[i] = narrow16x2<false>(widen16<true>(words[i] & 0xFFFFu), widen16<true>(words[i] >> 16));
-    return uint4{out[0], out[1], out[2], out[3]};
-}
-
-// the sum of squares of 8 raw values: fp16 pairs by v_dot2_f32_f16; bf16 widened, then f32 products in order
-template <bool BF16 = false> DEVICE float squares8(const uint4& w, float c) {
-    if constexpr (BF16) {
-        float v[8];
-        widen8<true>(w, v);
-#pragma unroll
-        for (int i = 0; i < 8; i++) c = __builtin_fmaf(v[i], v[i], c);
-        return c;
-    } else {
-        return dot2(w.w, w.w, dot2(w.z, w.z, dot2(w.y, w.y, dot2(w.x, w.x, c))));
-    }
-}
-// O^T += V^T P^T for one 32-key step: the raw values (fp16 or bf16) and P (already rounded to the same type), 8 a lane
-template <bool BF16> DEVICE v4f pv_step(const uint4& v, const uint4& p, v4f acc) {
-    if constexpr (BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, v), __builtin_bit_cast(bf8, p), acc, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, v), __builtin_bit_cast(v8h, p), acc, 0, 0, 0);
-}
-
-// P V's P: fp16 rows round P to fp16, the reference's rounding point (model/attention_cuda.py:236-293); bf16 rows take P
-// as a bf16 high part hi (P rounded) and low part lo = bf16(P - hi) (the subtraction exact), so that P V in bf16 carries
-// about 16 bits of P, not bf16's 8, and the output's error stays that of its own bf16 rounding. low_parts gives lo's words
-// for a step's 8 probabilities (two rows of 4) whose high words are hi; pv_steps adds V hi, then V lo, into acc.
-template <bool BF16> DEVICE uint4 low_parts(const uint32_t (&hi)[4], const float (&first)[4], const float (&second)[4]) {
-    if constexpr (BF16) {
-        uint32_t lo[4];
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            lo[r] = narrow16x2<true>(first[2 * r] - widen16<true>(hi[r] & 0xFFFFu), first[2 * r + 1] - widen16<true>(hi[r] >> 16));
-            lo[2 + r] = narrow16x2<true>(second[2 * r] - widen16<true>(hi[2 + r] & 0xFFFFu), second[2 * r + 1] - widen16<true>(hi[2 + r] >> 16));
-        }
-        return uint4{lo[0], lo[1], lo[2], lo[3]};
-    } else {
-        return uint4{0, 0, 0, 0};
-    }
-}
-template <bool BF16> DEVICE v4f pv_steps(const uint4& v, const uint4& hi, const uint4& lo, v4f acc) {
-    if constexpr (BF16) return pv_step<true>(v, lo, pv_step<true>(v, hi, acc));
-    else return pv_step<false>(v, hi, acc);
-}
-
-// a workgroup's threads: Layout::WAVES wavefronts
-template <int TILES, bool SPLIT> constexpr int attention_threads() { return 64 * (SPLIT ? 4 : TILES); }
-
 // TILES: key tiles of 16 the instantiation holds (T <= 16 TILES)
-template <int DQP, int DV, int TILES, bool SPLIT = false>
+template <int DQP, int DV, int TILES>
 struct Layout {
     static constexpr int STEPS = (TILES + 1) / 2;     // 32-key steps of P V
     static constexpr int KEYS = TILES * 16;           // keys (and queries) staged
     static constexpr int KC = DQP / 8, VC = DV / 8;   // 16-byte chunks a raw key (query) row, a raw value row
     // value keys staged, whole DMA instructions of them (64 chunks): a half step of P V past them reads zeros
     static constexpr int VKEYS = (KEYS * VC + 63) / 64 * 64 / VC;
-    // SPLIT (five tiles: 65 to 80 tokens, the network's 70): four wavefronts, one a slab of 16 square queries, and the
-    // slab of the tokens past the squares split over three of them by 32-key step of P V (its partial maxima, sums and
-    // outputs meet in LDS), so that a workgroup's wavefronts spread evenly over a compute unit's four SIMDs and two
-    // workgroups fit one. The work past the square slabs is spread so that no wavefront waits long at a barrier:
-    // wavefront 3 normalises keys 64 .. 79 and wavefront 1 the split slab's queries (once, in LDS, for the three part
-    // wavefronts) while wavefront 2 merges the previous group's parts. Else one wavefront a slab.
-    static constexpr bool META = SPLIT;
-    static_assert(!SPLIT || TILES == 5, "the split slab is the fifth");
-    static constexpr int WAVES = META ? 4 : TILES;
-    // With five tiles every slab's softmax sum and P V outputs are added by 32-key step, in step order, whichever
-    // wavefront holds them, so that both launches give a query the same bits.
-    static constexpr bool BY_STEP = TILES == 5;
-    static_assert(attention_threads<TILES, SPLIT>() == 64 * WAVES, "the launch bounds' threads");
-    // LDS in bytes: two buffers of keys (raw as they land, normalised in place), two of raw values, the partial results
-    // of the split slab, then two buffers of raw queries and template coefficients
+    static constexpr int WAVES = TILES;               // one a slab of 16 queries
+    // LDS in bytes: two buffers of keys (raw as they land, normalised in place), two of raw values, then
+    // two of raw queries and template coefficients
     static constexpr int RAW_K_BYTES = KEYS * DQP * 2;   // a buffer's
     static constexpr int RAW_V_BYTES = VKEYS * DV * 2;   // a buffer's
     static constexpr int RAW_Q_BYTES = KEYS * DQP * 2;   // a head's
     static constexpr int COEF_BYTES = 64 * MAX_TEMPLATES * 2;   // a head's template coefficients, a square query a row
-    static constexpr int META_PARTS = 3;                 // the split slab's 32-key steps, one a wavefront
-    static constexpr int META_OUT = 64 * (DV / 4);       // a part's outputs: a lane's DV / 16 fragments of 4 f32
-    static constexpr int META_BYTES = META ? META_PARTS * (2 * 16 + META_OUT) * 4 : 0;
-    static constexpr int FIXED_BYTES = 2 * RAW_K_BYTES + 2 * RAW_V_BYTES + META_BYTES;
+    static constexpr int FIXED_BYTES = 2 * RAW_K_BYTES + 2 * RAW_V_BYTES;
     static int bytes(int per_kv) { return FIXED_BYTES + 2 * per_kv * (RAW_Q_BYTES + COEF_BYTES); }
 };
 
-// Raw rows are DMA'd 64 16-byte chunks an instruction, the chunks of a row in a swizzled order: chunk c of row r
-// sits in slot r * CH + (c ^ swizzle(r)), which puts the 16 rows an MFMA operand group reads (one chunk each) in
-// 16 different 16-byte bank groups.
 // Every wavefront's LDS writes are done and visible; unlike __syncthreads, the DMA loads in flight go on.
 DEVICE void lds_barrier() {
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0), vmcnt and expcnt left alone
@@ -356,9 +53,6 @@ DEVICE void lds_barrier() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-
-template <int CH> DEVICE int swizzle(int row) { return CH >= 16 ? row % CH : (row / (16 / CH)) % CH; }
-template <int CH> DEVICE int raw_slot(int row, int chunk) { return row * CH + (chunk ^ swizzle<CH>(row)); }
 
 // A wavefront's share of the DMA of a raw block of ROWS rows x CH 16-byte chunks, 64 chunks an instruction:
 // instruction i = wave + j WAVES writes slots i * 64 + lane, slot s holding chunk (s % CH) ^ swizzle(row) of row
@@ -396,33 +90,27 @@ struct DmaPlan {
 // TILES = ceil(T / 16) exactly: the launch picks the instantiation, so every count below is fixed at compile time.
 // Registers are held to two wavefronts a SIMD, within which the query and value widths up to 64 need no scratch (a
 // scratch reload would wait for the DMA in flight too); query widths of 128, and value widths of 128 past 96 tokens,
-// spill some, and so does the split slab's bf16 instantiation (its P low parts). (Fewer registers for more workgroups
-// a CU cost more instructions than they gain: the kernel is bound by its VALU work.)
-// ONE_HEAD: one query head a key/value head (the network's heads == kv_heads), fixed at compile time: the loops over a
-// group's heads go, and with them the scalar registers they held and spilled (100.9 against 108.9 us at batch 1024,
-// 12.7 against 13.5 at batch 64, 70 tokens and 8 x 64 heads on an MI355X; the same bits).
-template <int DQP, int DV, int TILES, bool SPLIT, bool BF16, bool ONE_HEAD = false>
-__global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__((amdgpu_waves_per_eu(2))) void template_attention_kernel(
+// spill some. (Fewer registers for more workgroups a CU cost more instructions than they gain: the kernel is bound by its
+// VALU work.)
+template <int DQP, int DV, int TILES, bool BF16>
+__global__ __launch_bounds__(64 * TILES) __attribute__((amdgpu_waves_per_eu(2))) void template_attention_kernel(
     const half_t* __restrict__ projected, const half_t* __restrict__ keyed, const half_t* __restrict__ q_gain,
     const half_t* __restrict__ k_gain, half_t* __restrict__ out, int T, int heads, int kv_heads, int dq, int templates_count,
     int groups_per_block, float eps, float scale)
 {
-    typedef Layout<DQP, DV, TILES, SPLIT> L;
+    typedef Layout<DQP, DV, TILES> L;
+    constexpr bool BY_STEP = TILES == 5;   // with five tiles the softmax sum and P V outputs are added by 32-key step, in step order
     constexpr int KC = L::KC, VC = L::VC, WAVES = L::WAVES, THREADS = 64 * WAVES, STEPS = L::STEPS, KEYS = L::KEYS;
     extern __shared__ __align__(16) int8_t lds[];
     LDS_SPACE int8_t* raw_k = (LDS_SPACE int8_t*)lds;                        // [2][KEYS * DQP halves]
     LDS_SPACE int8_t* raw_v = raw_k + 2 * L::RAW_K_BYTES;                    // [2][VKEYS * DV halves]
-    // the split slab's parts: maxima [3][16], sums [3][16], outputs [3][64 lanes][DV / 4] (f32)
-    float* meta_max = (float*)(lds + 2 * L::RAW_K_BYTES + 2 * L::RAW_V_BYTES);
-    float* meta_sum = meta_max + L::META_PARTS * 16;
-    float* meta_out = meta_sum + L::META_PARTS * 16;
-    LDS_SPACE int8_t* raw_q = raw_v + 2 * L::RAW_V_BYTES + L::META_BYTES;    // [2][per_kv][KEYS * DQP halves]
+    LDS_SPACE int8_t* raw_q = raw_v + 2 * L::RAW_V_BYTES;    // [2][per_kv][KEYS * DQP halves]
     LDS_SPACE int8_t* raw_c = raw_q + 2 * (heads / kv_heads) * L::RAW_Q_BYTES;   // [2][per_kv][64][8 halves]
 
     const int tid = threadIdx.x, lane = tid & 63, slab = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int width = heads * dq + kv_heads * dq + kv_heads * DV + heads * templates_count;
     const int k_offset = heads * dq, v_offset = k_offset + kv_heads * dq, c_offset = v_offset + kv_heads * DV;
-    const int per_kv = ONE_HEAD ? 1 : heads / kv_heads;
+    const int per_kv = heads / kv_heads;
     // pair p of the launch is key/value group p % kv_heads of position p / kv_heads
     auto board_of = [&](int pair) { return projected + (size_t)(pair / kv_heads) * T * width; };
     const int first_pair = blockIdx.x * groups_per_block;
@@ -536,51 +224,6 @@ __global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__(
         }
     };
 
-    // The split slab (L::META): its queries 64 .. 79 are normalised once, in place in a head's query rows, by one
-    // wavefront in the layout and order the main slabs use (lane (col, quad) holds chunks quad and 4 + quad of its query;
-    // the rows' partial sums added as (r0 + r1) + (r2 + r3)), so the part wavefronts read the very q' they would compute.
-    const int meta_query = 64 + col;
-    auto normalise_meta_queries = [&](LDS_SPACE int8_t* queries) {
-        uint4 mraw[DQP / 32];
-        float msquares = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < DQP / 32; ks++) {
-            const int c = ks * 4 + quad;
-            mraw[ks] = lds_chunk(queries + raw_slot<KC>(meta_query, c) * 16);
-            if (c * 8 >= dq) mraw[ks] = uint4{0, 0, 0, 0};
-            msquares = squares8<BF16>(mraw[ks], msquares);
-        }
-        msquares = sum_across_rows(msquares);
-        const float inverse = inverse_norm(msquares);
-#pragma unroll
-        for (int ks = 0; ks < DQP / 32; ks++) {
-            v8h normed;
-            float wide[8];
-            widen8<BF16>(mraw[ks], wide);
-#pragma unroll
-            for (int e = 0; e < 8; e++) normed[e] = (half_t)((wide[e] * inverse) * gains[ks][e]);
-            *reinterpret_cast<LDS_SPACE v8h*>(queries + raw_slot<KC>(meta_query, ks * 4 + quad) * 16) = normed;
-        }
-    };
-    // The split slab's parts added in part order and written out, for one head of a pair: by wavefront 2, once the parts'
-    // sums and outputs are in LDS. The merge of a group's last head waits for the next group's first barrier, so that it
-    // runs beside the next group's key normalisation rather than after everything else.
-    auto merge = [&](int merge_pair, int head) {
-        if (meta_query >= T) return;
-        const float mtotal = (meta_sum[col] + meta_sum[16 + col]) + meta_sum[32 + col];
-        const float minverse = __builtin_amdgcn_rcpf(mtotal);
-        half_t* to = out + ((size_t)(merge_pair / kv_heads) * T + meta_query) * (heads * DV) + head * DV + quad * 4;
-#pragma unroll
-        for (int dt = 0; dt < DV / 16; dt++) {
-            const v4f p0 = *reinterpret_cast<const v4f*>(meta_out + lane * (DV / 4) + dt * 4);
-            const v4f p1 = *reinterpret_cast<const v4f*>(meta_out + L::META_OUT + lane * (DV / 4) + dt * 4);
-            const v4f p2 = *reinterpret_cast<const v4f*>(meta_out + 2 * L::META_OUT + lane * (DV / 4) + dt * 4);
-            float merged[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) merged[r] = ((p0[r] + p1[r]) + p2[r]) * minverse;
-            *reinterpret_cast<uint2*>(to + dt * 16) = uint2{narrow16x2<BF16>(merged[0], merged[1]), narrow16x2<BF16>(merged[2], merged[3])};
-        }
-    };
     // The templates and gains have landed before the loop (with the first group's rows): counting loads across the
     // loop's iterations, the compiler would otherwise wait for every load in flight -- the next group's rows too --
     // at each use of them in the loop.
@@ -601,8 +244,7 @@ __global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__(
 #pragma unroll
             for (int k = 0; k < O_ITEMS; k++) {
                 const int item = tid + k * THREADS, q = item / VC, c = item % VC;
-                // the split slab's rows (past the squares) are written by its merge, not staged
-                if ((O_TOTAL % THREADS == 0 || item < O_TOTAL) && q < (L::META ? min(T, 64) : T))
+                if ((O_TOTAL % THREADS == 0 || item < O_TOTAL) && q < T)
                     *reinterpret_cast<uint4*>(to + (size_t)q * (heads * DV) + c * 8) = lds_chunk(staged + raw_slot<KC>(q, c) * 16);
             }
         }
@@ -618,25 +260,11 @@ __global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__(
         __syncthreads();
 
         LDS_SPACE int8_t* group_keys = raw_k + buffer * L::RAW_K_BYTES;
-        if constexpr (L::META) {
-            // keys 0 .. 63 by every thread; then a wavefront each: keys 64 .. 79, the split slab's queries of each head,
-            // and the previous group's split slab merged (its parts landed before the barrier above)
-            static_assert(THREADS / 4 == 64, "the square keys in one pass");
-            normalise_key(group_keys, tid / 4);
-            if (slab == 3) {
-                normalise_key(group_keys, 64 + lane / 4);
-            } else if (slab == 1) {
-                for (int hi = 0; hi < per_kv; hi++) normalise_meta_queries(raw_q + (buffer * per_kv + hi) * head_bytes);
-            } else if (slab == 2 && gi > 0) {
-                merge(pair - 1, ((pair - 1) % kv_heads + 1) * per_kv - 1);
-            }
-        } else {
 #pragma unroll
-            for (int pass = 0; pass < KEY_PASSES; pass++) {
-                const int scale_key = pass * (THREADS / 4) + tid / 4;
-                if (KEYS * 4 % THREADS != 0 && scale_key >= KEYS) break;
-                normalise_key(group_keys, scale_key);
-            }
+        for (int pass = 0; pass < KEY_PASSES; pass++) {
+            const int scale_key = pass * (THREADS / 4) + tid / 4;
+            if (KEYS * 4 % THREADS != 0 && scale_key >= KEYS) break;
+            normalise_key(group_keys, scale_key);
         }
         // The previous group's outputs leave its query buffer once the keys are normalised; after the barrier every
         // wavefront has read its share, and the next group's keys, values and queries load into the other buffers. (Issued
@@ -737,7 +365,7 @@ __global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__(
             top = max_across_rows(top);
             float total = 0.0f;
             const float offset = -top * LOG2E;
-            if constexpr (L::BY_STEP) {
+            if constexpr (BY_STEP) {
                 // each 32-key step's sum across the wavefront, then the steps' sums in order
 #pragma unroll
                 for (int st = 0; st < STEPS; st++) {
@@ -800,7 +428,7 @@ __global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__(
 #pragma unroll
                 for (int dt = 0; dt < DV / 16; dt++) {
                     const uint4 vf = uint4{lower[dt][0], lower[dt][1], upper[dt][0], upper[dt][1]};
-                    if constexpr (L::BY_STEP && st > 0) {
+                    if constexpr (BY_STEP && st > 0) {
                         o[dt] = o[dt] + pv_steps<BF16>(vf, pf, pf_lo, v4f{0, 0, 0, 0});
                     } else {
                         o[dt] = pv_steps<BF16>(vf, pf, pf_lo, o[dt]);
@@ -825,157 +453,56 @@ __global__ __launch_bounds__((attention_threads<TILES, SPLIT>())) __attribute__(
                     *reinterpret_cast<uint2*>(to + dt * 16) = result;
                 }
             }
-
-            if constexpr (L::META) {
-                // The slab of queries 64..79 (the tokens past the squares: no template bias), split by 32-key step of
-                // P V: wavefronts 0, 1 and 3 take steps 0, 1 and 2 (key tiles 2p, 2p + 1), wavefront 2 adds their parts.
-                // Each part's maximum is exchanged first, so that every part's probabilities are f16(exp(s - the
-                // row's maximum)) as in the one-wavefront slab; the parts' sums and outputs are added in part order.
-                const int part = slab == 3 ? 2 : slab;   // wavefront 2: the merge
-                float ms[2][4];
-                if (slab != 2) {
-                    v8h mq[DQP / 32];   // normalised in place before the group's second barrier
-#pragma unroll
-                    for (int ks = 0; ks < DQP / 32; ks++)
-                        mq[ks] = *reinterpret_cast<const LDS_SPACE v8h*>(queries + raw_slot<KC>(meta_query, ks * 4 + quad) * 16);
-                    float mtop = -__builtin_inff();
-#pragma unroll
-                    for (int h2 = 0; h2 < 2; h2++) {
-                        const int kt = 2 * part + h2;
-                        if (kt >= TILES) {
-#pragma unroll
-                            for (int r = 0; r < 4; r++) ms[h2][r] = -__builtin_inff();
-                            continue;
-                        }
-                        v4f acc = v4f{0, 0, 0, 0};
-#pragma unroll
-                        for (int ks = 0; ks < DQP / 32; ks++) {
-                            const v8h kf = *reinterpret_cast<const LDS_SPACE v8h*>(keys + raw_slot<KC>(kt * 16 + col, ks * 4 + quad) * 16);
-                            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, mq[ks], acc, 0, 0, 0);
-                        }
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const float value = kt * 16 + quad * 4 + r >= T ? -__builtin_inff() : acc[r] * scale;
-                            ms[h2][r] = value;
-                            mtop = fmaxf(mtop, value);
-                        }
-                    }
-                    mtop = max_across_rows(mtop);
-                    if (quad == 0) meta_max[part * 16 + col] = mtop;
-                }
-                lds_barrier();   // the parts' maxima are in place
-                if (slab != 2) {
-                    const float top_all = fmaxf(fmaxf(meta_max[col], meta_max[16 + col]), meta_max[32 + col]);
-                    const float moffset = -top_all * LOG2E;
-                    float mtotal = 0.0f;
-#pragma unroll
-                    for (int h2 = 0; h2 < 2; h2++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const float p = 2 * part + h2 < TILES ? __builtin_amdgcn_exp2f(__builtin_fmaf(ms[h2][r], LOG2E, moffset)) : 0.0f;
-                            ms[h2][r] = p;
-                            mtotal += p;
-                        }
-                    mtotal = sum_across_rows(mtotal);
-                    if (quad == 0) meta_sum[part * 16 + col] = mtotal;
-                    uint32_t pw[4];
-#pragma unroll
-                    for (int r = 0; r < 2; r++) {
-                        pw[r] = narrow16x2<BF16>(ms[0][2 * r], ms[0][2 * r + 1]);
-                        pw[2 + r] = narrow16x2<BF16>(ms[1][2 * r], ms[1][2 * r + 1]);
-                    }
-                    const uint4 pf = uint4{pw[0], pw[1], pw[2], pw[3]};
-                    const uint4 pf_lo = low_parts<BF16>(pw, ms[0], ms[1]);
-                    constexpr int ROW_BYTES = VC * 16;
-                    const int lo_rows = 32 * part * ROW_BYTES, hi_rows = (32 * part + 16) * ROW_BYTES;
-                    const bool has_hi = 32 * part + 16 < L::VKEYS;
-                    // both halves read (without the upper keys, the lower ones again), then the upper zeroed
-                    uint32_t lower_at[DV / 16], upper_at[DV / 16];
-#pragma unroll
-                    for (int dt = 0; dt < DV / 16; dt++) {
-                        lower_at[dt] = value_words[dt] + lo_rows;
-                        upper_at[dt] = value_words[dt] + (has_hi ? hi_rows : lo_rows);
-                    }
-                    v2u lower[DV / 16], upper[DV / 16];
-                    part_reads<DV / 16>(lower_at, upper_at, lower, upper);
-                    float* mine = meta_out + part * L::META_OUT + lane * (DV / 4);
-#pragma unroll
-                    for (int dt = 0; dt < DV / 16; dt++) {
-                        if (!has_hi) upper[dt] = v2u{0, 0};
-                        const uint4 vf = uint4{lower[dt][0], lower[dt][1], upper[dt][0], upper[dt][1]};
-                        const v4f partial = pv_steps<BF16>(vf, pf, pf_lo, v4f{0, 0, 0, 0});
-                        *reinterpret_cast<v4f*>(mine + dt * 4) = partial;
-                    }
-                }
-                if (hi + 1 < per_kv) {
-                    // the next head's parts reuse the LDS: merged now (the group's last head is merged after the next
-                    // group's first barrier)
-                    lds_barrier();   // the parts' sums and outputs are in place
-                    if (slab == 2) merge(pair, head);
-                }
-            }
         }
     }
-    if constexpr (STAGED || L::META) {
-        __builtin_amdgcn_s_waitcnt(0);   // this wavefront's staging and part writes are done (the compiler does not see them)
+    if constexpr (STAGED) {
+        __builtin_amdgcn_s_waitcnt(0);   // this wavefront's staging writes are done (the compiler does not see them)
         __syncthreads();
-        const int last = first_pair + groups_per_block - 1;
-        if constexpr (STAGED) write_out(last, (groups_per_block - 1) & 1);
-        if constexpr (L::META)
-            if (slab == 2) merge(last, (last % kv_heads + 1) * per_kv - 1);
+        write_out(first_pair + groups_per_block - 1, (groups_per_block - 1) & 1);
     }
 }
 
-template <int DQP, int DV, int TILES, bool SPLIT, bool BF16, bool ONE_HEAD = false>
+template <int DQP, int DV, int TILES, bool BF16>
 int launch(const void* projected, const void* keyed, const void* q_gain, const void* k_gain, void* out, int B, int T, int heads,
            int kv_heads, int dq, int templates_count, int groups_per_block, float eps, float scale, hipStream_t stream)
 {
-    typedef Layout<DQP, DV, TILES, SPLIT> L;
+    typedef Layout<DQP, DV, TILES> L;
+    // (refused whichever kernel runs, so that what the operator takes does not depend on the tokens)
     const int bytes = L::bytes(heads / kv_heads);
     if (bytes > 160 * 1024)
         return chess_fail(CHESS_UNSUPPORTED, "template_attention would stage %d bytes of LDS for %d heads a key/value head", bytes, heads / kv_heads);
-    auto kernel = template_attention_kernel<DQP, DV, TILES, SPLIT, BF16, ONE_HEAD>;
-    if (bytes > 65536) {
-        const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        if (allowed != hipSuccess) return (int)allowed;
-    }
-    const dim3 grid((unsigned)((long)B * kv_heads / groups_per_block)), block(64 * L::WAVES);   // TILES == ceil(T / 16): the caller picked it so
-    // (bf16 rows travel as 16-bit elements behind the same pointers: the kernel reads them only through widen16<BF16>)
-    hipLaunchKernelGGL(kernel, grid, block, bytes, stream, (const half_t*)projected, (const half_t*)keyed, (const half_t*)q_gain,
-                       (const half_t*)k_gain, (half_t*)out, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale);
-    return launch_status();
-}
-
-// ONE_HEAD (heads == kv_heads) instantiated for 64 to 80 tokens, the network's 70 and the benchmark's 64
-template <int DQP, int DV, bool BF16, bool ONE_HEAD>
-int by_tokens(const void* projected, const void* keyed, const void* q_gain, const void* k_gain, void* out, int B, int T, int heads,
-              int kv_heads, int dq, int templates_count, int groups_per_block, float eps, float scale, hipStream_t stream)
-{
-    switch ((T + 15) / 16) {
-        case 4: return launch<DQP, DV, 4, false, BF16, ONE_HEAD>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-        case 5:
-            // four wavefronts a workgroup (the split slab) once the launch has pairs to keep two workgroups on each compute
-            // unit busy: at 70 tokens and 8 x 64 heads on an MI355X, each at its best run of pairs a workgroup, batch 1024
-            // in 108 against 122.0 us, batch 512 in 62.5 against 65.0, batch 256 32.4 against 36.2, batch 128 20.6 against
-            // 22.0; batch 64 13.6 either way, batch 32 10.9 against 9.7. Query and value widths up to 64: past them the split
-            // slab's registers spill.
-            if constexpr (DQP <= 64 && DV <= 64)
-                if ((long)B * kv_heads >= SPLIT_PAIRS)
-                    return launch<DQP, DV, 5, true, BF16, ONE_HEAD>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-            return launch<DQP, DV, 5, false, BF16, ONE_HEAD>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-        case 6: return launch<DQP, DV, 6, false, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-        case 7: return launch<DQP, DV, 7, false, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-        default: return launch<DQP, DV, 8, false, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
+    // widths up to 64 and up to 80 tokens: attention_wave.h's kernel, which shares the pairs out by itself
+    if constexpr (DQP <= 64 && DV <= 64 && TILES <= 5) {
+        return launch_waves<DQP, DV, TILES, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, eps, scale, stream);
+    } else {
+        auto kernel = template_attention_kernel<DQP, DV, TILES, BF16>;
+        if (bytes > 65536) {
+            const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+            if (allowed != hipSuccess) return (int)allowed;
+        }
+        const dim3 grid((unsigned)((long)B * kv_heads / groups_per_block)), block(64 * L::WAVES);   // TILES == ceil(T / 16): the caller picked it so
+        // (bf16 rows travel as 16-bit elements behind the same pointers: the kernel reads them only through widen16<BF16>)
+        hipLaunchKernelGGL(kernel, grid, block, bytes, stream, (const half_t*)projected, (const half_t*)keyed, (const half_t*)q_gain,
+                           (const half_t*)k_gain, (half_t*)out, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale);
+        return launch_status();
     }
 }
 
 template <int DQP, int DV, bool BF16>
-int by_heads(const void* projected, const void* keyed, const void* q_gain, const void* k_gain, void* out, int B, int T, int heads,
-             int kv_heads, int dq, int templates_count, int groups_per_block, float eps, float scale, hipStream_t stream)
+int by_tokens(const void* projected, const void* keyed, const void* q_gain, const void* k_gain, void* out, int B, int T, int heads,
+              int kv_heads, int dq, int templates_count, int groups_per_block, float eps, float scale, hipStream_t stream)
 {
-    if constexpr (DQP <= 64 && DV <= 64)
-        if (heads == kv_heads) return by_tokens<DQP, DV, BF16, true>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-    return by_tokens<DQP, DV, BF16, false>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
+    auto launched = [&](auto tiles) {
+        return launch<DQP, DV, decltype(tiles)::value, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count,
+                                                             groups_per_block, eps, scale, stream);
+    };
+    switch ((T + 15) / 16) {
+        case 4: return launched(std::integral_constant<int, 4>{});
+        case 5: return launched(std::integral_constant<int, 5>{});
+        case 6: return launched(std::integral_constant<int, 6>{});
+        case 7: return launched(std::integral_constant<int, 7>{});
+        default: return launched(std::integral_constant<int, 8>{});
+    }
 }
 
 template <int DQP, bool BF16>
@@ -983,12 +510,12 @@ int by_dv(const void* projected, const void* keyed, const void* q_gain, const vo
           int kv_heads, int dq, int dv, int templates_count, int groups_per_block, float eps, float scale, hipStream_t stream)
 {
     switch (dv) {
-        case 16: return by_heads<DQP, 16, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-        case 32: return by_heads<DQP, 32, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
-        case 64: return by_heads<DQP, 64, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
+        case 16: return by_tokens<DQP, 16, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
+        case 32: return by_tokens<DQP, 32, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
+        case 64: return by_tokens<DQP, 64, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
         default:
             if constexpr (BF16) return chess_fail(CHESS_UNSUPPORTED, "template_attention takes bf16 rows of value widths up to 64");
-            else return by_heads<DQP, 128, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
+            else return by_tokens<DQP, 128, BF16>(projected, keyed, q_gain, k_gain, out, B, T, heads, kv_heads, dq, templates_count, groups_per_block, eps, scale, stream);
     }
 }
 

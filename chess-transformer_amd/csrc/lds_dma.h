@@ -31,9 +31,17 @@ DEVICE void buffer_dma16(BufferResource resource, LDS_SPACE void* to, uint32_t l
 DEVICE void buffer_dma4(BufferResource resource, LDS_SPACE void* to, uint32_t lane_offset, uint32_t offset) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(resource, to, 4, lane_offset, offset, 0, 0);
 }
+// the same, 16 bytes a lane, streamed past the caches (non-temporal)
+DEVICE void buffer_dma16_streamed(BufferResource resource, LDS_SPACE void* to, uint32_t lane_offset, uint32_t offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(resource, to, 16, lane_offset, offset, 0, 2);
+}
 // 16 bytes a lane from a buffer into registers, the lane's offset from a VGPR and a uniform offset from an SGPR
 DEVICE uint4 buffer_load16(BufferResource resource, uint32_t lane_offset, uint32_t offset) {
     const v4u v = __builtin_amdgcn_raw_buffer_load_b128(resource, lane_offset, offset, 0);
+    return uint4{v[0], v[1], v[2], v[3]};
+}
+DEVICE uint4 buffer_load16_streamed(BufferResource resource, uint32_t lane_offset, uint32_t offset) {   // non-temporal
+    const v4u v = __builtin_amdgcn_raw_buffer_load_b128(resource, lane_offset, offset, 2);
     return uint4{v[0], v[1], v[2], v[3]};
 }
 // 8 and 4 bytes a lane from a buffer into registers (zeros past the resource's bytes)
@@ -63,7 +71,9 @@ struct BufferResource {};
 DEVICE BufferResource buffer_resource(const void*, uint32_t) { return {}; }
 DEVICE void buffer_dma16(BufferResource, LDS_SPACE void*, uint32_t, uint32_t) {}
 DEVICE void buffer_dma4(BufferResource, LDS_SPACE void*, uint32_t, uint32_t) {}
+DEVICE void buffer_dma16_streamed(BufferResource, LDS_SPACE void*, uint32_t, uint32_t) {}
 DEVICE uint4 buffer_load16(BufferResource, uint32_t, uint32_t) { return uint4{0, 0, 0, 0}; }
+DEVICE uint4 buffer_load16_streamed(BufferResource, uint32_t, uint32_t) { return uint4{0, 0, 0, 0}; }
 DEVICE uint2 buffer_load8(BufferResource, uint32_t, uint32_t) { return uint2{0, 0}; }
 DEVICE uint32_t buffer_load4(BufferResource, uint32_t, uint32_t) { return 0; }
 DEVICE void buffer_store8(BufferResource, uint2, uint32_t, uint32_t) {}

@@ -43,10 +43,9 @@ LINEAR_F32_TILES = {"gfx950": [(4, 1), (math.inf, 7)]}
 # 22.0 / 57.6 against 23.8 / 58.0 us) and 64 x 64 up to 9 (batch 16: 11.8 against 20.7 us)
 LINEAR_LONG_ROW_TILES = {"gfx950": [(9, 1), (160, 12), (math.inf, 13)]}
 LONG_ROW_BYTES = 2048
-# from this many (position, key/value group) pairs a template_attention launch of 65 to 80 tokens, query and value widths
-# up to 64, splits the slab of the tokens past the squares over three wavefronts: workgroups of four wavefronts instead
-# of five (the kernel's SPLIT_PAIRS). Timed on an MI355X at 70 tokens and 8 x 64 heads, each at its best run of pairs: batch
-# 256 34.4 us split against 41.4 us, batch 128 20.6 against 22.0, batch 64 13.6 either way, batch 32 10.9 against 9.7
+# from this many (position, key/value group) pairs groups_per_workgroup plans a launch of 65 to 80 tokens, query and value
+# widths up to 64, for workgroups of four wavefronts instead of five. (Such launches, and those of 64 tokens, share their pairs
+# out by themselves and only check that the run divides them: csrc/attention_wave.h.)
 ATTENTION_SPLIT_PAIRS = 1024
 
 
@@ -74,7 +73,8 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
 
 
 def attention_waves(positions: int, kv_heads: int, tokens: int, dq: int, dv: int) -> int:
-    """A template_attention workgroup's wavefronts: one a slab of 16 queries, or four for the split slab."""
+    """The wavefronts that a template_attention workgroup is planned with: one a slab of 16 queries, or four in launches of
+    ATTENTION_SPLIT_PAIRS on, where the fifth slab is one of the four's too."""
     tiles = (tokens + 15) // 16
     split = tiles == 5 and dq <= 64 and dv <= 64 and positions * kv_heads >= ATTENTION_SPLIT_PAIRS
     return 4 if split else tiles
@@ -84,9 +84,8 @@ def groups_per_workgroup(positions: int, kv_heads: int, multiprocessors: int = 2
     """The most (position, key/value group) pairs a workgroup takes -- a divisor of all the launch's pairs -- while the launch
     keeps as many workgroups as the compute units hold at once (two wavefronts a SIMD, four SIMDs: one workgroup of five to
     eight wavefronts, two of four), so that a workgroup's start (its template registers and first loads) is paid once for
-    its pairs; any choice gives the same bits. Timed on an MI355X at 70 tokens and 8 x 64 heads: batch 16 at one pair a
-    workgroup, batch 64 at 256 workgroups of 2 pairs (13.7 us), batch 1024 at 512 of 16 (117.5 us; 256 of 32 in 122.0
-    and 1,024 of 8 in 137.7 before the split slab)."""
+    its pairs; any choice gives the same bits. It is what heads wider than 64 and more than 80 tokens run with; the others
+    balance themselves, which no divisor can: 24 on 12 heads at batch 700 had 525 workgroups of 16 pairs for 512 places."""
     pairs = positions * kv_heads
     workgroups = multiprocessors * max(1, 8 // attention_waves(positions, kv_heads, tokens, dq, dv))
     groups = max(1, pairs // workgroups)

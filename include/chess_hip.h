@@ -92,7 +92,8 @@ int chess_rotated_int8_linear(const void* h, const void* block_absmax, const voi
  * fp16, keyed_templates[64, 64, 8] fp16 (keyed[i][j][t] = templates[t][i][j] for t < tc, zero beyond; 16-byte
  * aligned), q_gain/k_gain[dq] fp16 -> out[B, T, H*dv] fp16; scale = 1/sqrt(dq).
  * A workgroup takes groups_per_block (position, key/value group) pairs in a row, which may run across positions
- * (any divisor of B * KV; it changes no bit).
+ * (any divisor of B * KV; it changes no bit). Up to 80 tokens with dq and dv up to 64 the launch shares its pairs out by
+ * itself, and groups_per_block is only checked.
  * Replaces template_attention_cuda (model/attention_cuda.py:97-304, launch :379-391, pointer order
  * projected, paired templates, q_gain, k_gain, out; templates paired once, :410-440) and the Triton pair
  * template_bias_kernel + template_attention_kernel (model/fused_blocks.py:35-171). */

@@ -684,6 +684,33 @@ def test_the_split_slab_launch_gives_the_small_launchs_bits(device, heads, kv_he
     assert torch.equal(few, split)
 
 
+@pytest.mark.parametrize("heads, kv_heads, dq, dv, tokens, count, positions", [
+    (8, 8, 64, 64, 70, 8, 129), (8, 8, 64, 64, 64, 8, 65), (4, 4, 40, 64, 66, 6, 257), (24, 12, 24, 32, 70, 8, 129), (8, 4, 8, 16, 80, 3, 385),
+    (2, 1, 32, 32, 65, 8, 1537)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_both_sharings_of_the_pairs_give_the_same_bits(device, heads, kv_heads, dq, dv, tokens, count, positions, dtype):
+    """Widths up to 64 and up to 80 tokens: a launch just past four pairs a compute unit (two over 64 tokens; six of widths up
+    to 32) gives its wavefronts whole pairs, and one of a few positions shares a pair over four. The same bits, the fp32
+    formula's answer, at the smallest and largest token counts, query widths that do not fill their chunks and fewer than
+    eight templates; a position of infinities and NaNs stays its own."""
+    projected, *rest = attention_operands(device, positions, heads, kv_heads, dq, dv, seed=tokens + dq, tokens=tokens, templates_count=count)
+    projected = projected.to(dtype)
+    arguments = (projected, *rest)
+    whole = template_attention(*arguments)
+    assert (whole.float() - reference_attention(arguments)).abs().max() < 1e-2
+    some = [0, 1, 2, positions // 2, positions - 2, positions - 1]
+    assert torch.equal(template_attention(projected[some].contiguous(), *arguments[1:]), whole[some])
+    spoilt = projected.clone()
+    spoilt[1] = float("nan")
+    spoilt[positions - 2, :, ::3] = float("inf")
+    clean = [position for position in range(positions) if position not in (1, positions - 2)]
+    for boards in (positions, 5):
+        rows = list(range(boards - 3)) + list(range(positions - 3, positions))
+        kept = [k for k, position in enumerate(rows) if position in set(clean)]
+        out = template_attention(spoilt[rows].contiguous(), *arguments[1:])
+        assert torch.equal(out[kept], whole[[rows[k] for k in kept]])
+
+
 def bf16_operands(arguments):
     projected, templates, *rest = arguments
     return (projected.bfloat16(), templates, *rest)
