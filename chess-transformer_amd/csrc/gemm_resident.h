@@ -114,8 +114,7 @@ template <> DEVICE uint2 pack_four<half_t>(const float (&v)[4]) {
     return __builtin_bit_cast(uint2, four);
 }
 template <> DEVICE uint2 pack_four<bf16_t>(const float (&v)[4]) {
-    return uint2{(uint32_t)bf16_from_float(v[0]).bits | ((uint32_t)bf16_from_float(v[1]).bits << 16),
-                 (uint32_t)bf16_from_float(v[2]).bits | ((uint32_t)bf16_from_float(v[3]).bits << 16)};
+    return uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
 }
 
 template <typename In, int NB, typename OutT, int EPI>

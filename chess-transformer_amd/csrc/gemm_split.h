@@ -39,7 +39,7 @@ template <> DEVICE void store_eight<half_t>(half_t* to, const float (&v)[8]) {
 template <> DEVICE void store_eight<bf16_t>(bf16_t* to, const float (&v)[8]) {
     v4u_t packed;
 #pragma unroll
-    for (int c = 0; c < 4; c++) packed[c] = (uint32_t)bf16_from_float(v[2 * c]).bits | ((uint32_t)bf16_from_float(v[2 * c + 1]).bits << 16);
+    for (int c = 0; c < 4; c++) packed[c] = bf16_pair(v[2 * c], v[2 * c + 1]);
     __builtin_nontemporal_store(packed, reinterpret_cast<v4u_t*>(to));
 }
 

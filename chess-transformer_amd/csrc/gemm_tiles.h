@@ -77,7 +77,7 @@ template <> DEVICE void store_eight<half_t>(half_t* to, const float (&v)[8]) {
 template <> DEVICE void store_eight<bf16_t>(bf16_t* to, const float (&v)[8]) {
     v4u packed;
 #pragma unroll
-    for (int c = 0; c < 4; c++) packed[c] = (uint32_t)bf16_from_float(v[2 * c]).bits | ((uint32_t)bf16_from_float(v[2 * c + 1]).bits << 16);
+    for (int c = 0; c < 4; c++) packed[c] = bf16_pair(v[2 * c], v[2 * c + 1]);
     __builtin_nontemporal_store(packed, reinterpret_cast<v4u*>(to));
 }
 template <> DEVICE void store_eight<float>(float* to, const float (&v)[8]) {
@@ -90,8 +90,8 @@ template <> DEVICE void stage_four<half_t>(half_t* to, const float (&v)[4]) {
     *reinterpret_cast<v4h*>(to) = v4h{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
 }
 template <> DEVICE void stage_four<bf16_t>(bf16_t* to, const float (&v)[4]) {
-    const uint32_t lo = (uint32_t)bf16_from_float(v[0]).bits | ((uint32_t)bf16_from_float(v[1]).bits << 16);
-    const uint32_t hi = (uint32_t)bf16_from_float(v[2]).bits | ((uint32_t)bf16_from_float(v[3]).bits << 16);
+    const uint32_t lo = bf16_pair(v[0], v[1]);
+    const uint32_t hi = bf16_pair(v[2], v[3]);
     *reinterpret_cast<uint2*>(to) = uint2{lo, hi};
 }
 template <typename OutT> DEVICE void stage_four(OutT*, const float (&)[4]) {}
