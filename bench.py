@@ -410,11 +410,14 @@ def kernel_role(name: str) -> str:
             return "fp16 block gate_up"
         return {"3": "combine (fp16, bias + residual)", "1": "fp16 block projection", "2": "fp16 block down",
                 "6": "fp16 block down (mix)"}.get(epilogue, "fp16 gemm")
-    if "resident_kernel" in name:   # template arguments In, NB, OutT, EPI
+    if "resident_kernel" in name:   # template arguments In, NB, OutT, EPI, depth
         found = re.search(r"resident_kernelI(a|DF16_)Li(\d)E(?:DF16_|DF16b)Li(\d)E", name)
         if found and found.group(1) == "DF16_":
             return "fp16 block projection (weights in registers)" if found.group(3) == "1" else "combine (fp16, bias + residual, weights in registers)"
-        return "gate_up (int8, gated, weights in registers)" if found and found.group(2) == "2" else "projection (int8, weights in registers)"
+        if found and found.group(2) == "2":
+            return "gate_up (int8, gated, weights in registers)"
+        return {"2": "down (int8, weights in registers)", "6": "down (int8, mixes the next input, weights in registers)"}.get(
+            found.group(3) if found else "", "projection (int8, weights in registers)")
     if "deep_kernel" in name:   # template arguments OutT, EPI
         found = re.search(r"deep_kernelI(?:DF16_|DF16b)Li(\d)E", name)
         return "down (int8, mixes the next input, weights in registers)" if found and found.group(1) == "6" else "down (int8, weights in registers)"

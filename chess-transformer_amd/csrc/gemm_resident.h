@@ -1,9 +1,11 @@
-// The GEMM of depth 512 with the weights held in registers (tile 15): out[M, N] = epilogue(x[M, 512] @ w[N, 512]^T), for
-// int8 operands (int32 sums) and for fp16 ones (f32 sums), with gemm_tiles.h's epilogues and op order (dequantise, bias,
-// SiLU * up, residual, round), so that it gives the other tiles' bits.
+// The GEMM with the weights held in registers: out[M, N] = epilogue(x[M, K] @ w[N, K]^T), for int8 operands (int32 sums, K =
+// 256, 512, 768 or 1,024) and for fp16 ones (f32 sums, K = 256 or 512), with gemm_tiles.h's epilogues and op order
+// (dequantise, bias, SiLU * up, residual, the next block's mix, round), so that it gives the other tiles' bits. Depth 512 is
+// tile 15; the others are launched by tile 0 alone.
 //
-// A wavefront owns 32 output columns and holds their weights for the whole depth in 128 VGPRs: int8, two fragments of 32
-// weight rows (gated: the gate's 32 rows and up's 32; else 64 columns), fp16, one. A workgroup of eight wavefronts (two a
+// A wavefront owns 32 output columns and holds their weights for the whole depth in up to 128 VGPRs: int8 up to depth 512, two
+// fragments of 32 weight rows (gated: the gate's 32 rows and up's 32; else 64 columns); int8 past it and fp16, one (gated:
+// 16 of the gate's rows and 16 of up's, whose sums meet in a lane too). A workgroup of eight wavefronts (two a
 // SIMD, one workgroup a compute unit) owns a column group of 256 (or 512) columns and walks a stream of 32-row blocks of
 // x, each block (16 KB of int8, 32 KB of fp16) arriving by DMA into a ring of four LDS stages: per block, every wavefront
 // reads the block's operands from LDS and runs its MFMAs into one of two sets of sums, while the epilogue of the block
@@ -34,7 +36,7 @@ using namespace gemm;
 typedef int v16i_r __attribute__((ext_vector_type(16)));
 typedef float v16f_r __attribute__((ext_vector_type(16)));
 
-constexpr int DEPTH = 512;      // K
+constexpr int DEPTH = 512;      // tile 15's K; tile 0 also takes the kernel's other depths (takes)
 constexpr int ROWS = 32;        // rows of x a block
 constexpr int WAVES = 8;
 constexpr int STAGES = 4;
@@ -54,22 +56,23 @@ template <> struct Mma<half_t> {
     static DEVICE float value(Sums c, int r) { return c[r]; }
 };
 
-template <typename In, int NB, int EPI> struct Shape {
+template <typename In, int NB, int EPI, int DEPTH_> struct Shape {
     static constexpr bool INT8 = std::is_same<In, int8_t>::value;
-    static constexpr bool BIAS = (EPI & EPI_BIAS) != 0, RESIDUAL = (EPI & EPI_RESIDUAL) != 0;
-    static constexpr int ROW_BYTES = DEPTH * (int)sizeof(In);      // 512 or 1024
+    static constexpr bool BIAS = (EPI & EPI_BIAS) != 0, RESIDUAL = (EPI & EPI_RESIDUAL) != 0, MIX = (EPI & EPI_MIX) != 0;
+    static constexpr int ROW_BYTES = DEPTH_ * (int)sizeof(In);     // 256 to 1,024, a multiple of 256
     static constexpr int STEPS = ROW_BYTES / 32;                    // MFMA steps
     static constexpr int CHUNKS = ROW_BYTES / 16;                   // 16-byte chunks a row
     static constexpr int BLOCK_BYTES = ROWS * ROW_BYTES;
-    static constexpr int FRAGMENTS = INT8 ? 2 : 1;                  // weight fragments of 32 rows a wavefront holds
-    static constexpr int OUTPUTS = NB == 2 ? 1 : FRAGMENTS;         // output fragments (gated: gate and up make one)
-    static constexpr int COLUMNS = 32 * OUTPUTS;                    // output columns a wavefront
+    // weight fragments of 32 rows a wavefront holds: two while they fit in 128 VGPRs beside the sums, so that an operand read
+    // from LDS serves two MFMAs; else one (gated: 16 of the gate's rows and 16 of up's)
+    static constexpr int FRAGMENTS = INT8 && ROW_BYTES <= 512 ? 2 : 1;
+    static constexpr int COLUMNS = 32 * FRAGMENTS / NB;             // output columns a wavefront
+    static constexpr int PER_LANE = COLUMNS / 2;                    // outputs a lane
     static constexpr int GROUP = WAVES * COLUMNS;                   // a workgroup's column group
-    static constexpr int ROWS_PER_DMA = 1024 / ROW_BYTES;
-    static constexpr int ROW_DMA = ROWS / WAVES / ROWS_PER_DMA;     // a wavefront's 1 KB DMA instructions a block
+    static constexpr int ROW_DMA = BLOCK_BYTES / 1024 / WAVES;      // a wavefront's 1 KB DMA instructions a block
     static constexpr int DMA_OPS = ROW_DMA + (INT8 ? 1 : 0);        // and (int8) the block's row scales
     static constexpr int STORE_OPS = COLUMNS / 16;                  // a wavefront's 16-byte stores a block
-    static constexpr int LOAD_OPS = RESIDUAL ? COLUMNS / 16 : 0;    // and its 16-byte residual loads
+    static constexpr int LOAD_OPS = (RESIDUAL ? COLUMNS / 16 : 0) + (MIX ? COLUMNS / 16 : 0);   // and its 16-byte residual and input loads
     // LDS: the ring's stages, (int8) each stage's row scales, a copy a wavefront, a word a lane, then each wavefront's
     // column vectors (64 weight scales, 64 biases)
     static constexpr int SCALE_BYTES = WAVES * 64 * 4;
@@ -87,7 +90,7 @@ template <typename In, int NB, int EPI> struct Shape {
         for (int t = issuing + 1 > 0 ? issuing + 1 : 0; t < b; t++) ops += DMA_OPS + (t >= 1 ? STORE_OPS + LOAD_OPS : 0);
         return ops;
     }
-    static_assert(ROW_DMA >= 1 && STORE_OPS >= 1, "shape");
+    static_assert(ROW_BYTES % 256 == 0 && ROW_BYTES <= 1024 && STORE_OPS >= 1 && (RESIDUAL || !MIX) && !(NB == 2 && RESIDUAL), "shape");
 };
 
 // A lane's 4-column groups q = 2 p and 2 p + 1 (columns 8 q + 4 (l / 32) ..), packed, traded between lanes l and l + 32
@@ -117,15 +120,15 @@ template <> DEVICE uint2 pack_four<bf16_t>(const float (&v)[4]) {
     return uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
 }
 
-template <typename In, int NB, typename OutT, int EPI>
+template <typename In, int NB, typename OutT, int EPI, int DEPTH_>
 __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
     const In* __restrict__ x, const In* __restrict__ w, OutT* __restrict__ out, Epilogue e, int M, int N, int groups, int slices,
     int last_slices)
 {
-    typedef Shape<In, NB, EPI> S;
+    typedef Shape<In, NB, EPI, DEPTH_> S;
     typedef Mma<In> MMA;
     typedef typename MMA::Operand Operand;
-    constexpr int STEPS = S::STEPS, ROW_BYTES = S::ROW_BYTES, FRAGMENTS = S::FRAGMENTS, OUTPUTS = S::OUTPUTS;
+    constexpr int STEPS = S::STEPS, ROW_BYTES = S::ROW_BYTES, FRAGMENTS = S::FRAGMENTS, COLUMNS = S::COLUMNS;
     extern __shared__ __align__(16) int8_t lds[];
     LDS_SPACE int8_t* ring = (LDS_SPACE int8_t*)lds;
 
@@ -154,7 +157,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
     Operand weights[FRAGMENTS][STEPS];
 #pragma unroll
     for (int f = 0; f < FRAGMENTS && !idle; f++) {
-        const int row = NB == 2 ? f * N + min(n_wave + in_row, N - 1) : min(n_wave + 32 * f + in_row, N - 1);
+        const int at_row = 32 * f + in_row;   // of the wavefront's weight rows: gated, the gate's COLUMNS, then up's
+        const int row = NB == 2 ? at_row / COLUMNS * N + min(n_wave + at_row % COLUMNS, N - 1) : min(n_wave + at_row, N - 1);
 #pragma unroll
         for (int t = 0; t < STEPS; t++)
             weights[f][t] = __builtin_bit_cast(Operand, buffer_load16(w_rsrc, (uint32_t)row * ROW_BYTES + 16 * half, 32 * t));
@@ -168,10 +172,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
     auto issue_one = [&](int b, int stage, int i) {   // DMA instruction i of block b into stage `stage`
         const int m0 = (first + b) * ROWS;
         if (i < S::ROW_DMA) {
-            const int rows_at = (ROWS / WAVES) * wave + S::ROWS_PER_DMA * i;
-            const int row = rows_at + lane / S::CHUNKS, slot = lane % S::CHUNKS;
+            const int instruction = S::ROW_DMA * wave + i, at_slot = instruction * 64 + lane;
+            const int row = at_slot / S::CHUNKS, slot = at_slot % S::CHUNKS;
             const uint32_t source = (uint32_t)min(m0 + row, M - 1) * ROW_BYTES + ((slot ^ (row & 15)) * 16);
-            buffer_dma16(x_rsrc, (LDS_SPACE void*)(ring + stage * S::BLOCK_BYTES + rows_at * ROW_BYTES), source, 0);
+            buffer_dma16(x_rsrc, (LDS_SPACE void*)(ring + stage * S::BLOCK_BYTES + instruction * 1024), source, 0);
         } else {   // lane l brings row l % 32's scale (no branch around the instruction)
             buffer_dma4(scale_rsrc, (LDS_SPACE void*)(ring + S::SCALES_AT + stage * S::SCALE_BYTES + 256 * wave),
                         (uint32_t)min(m0 + in_row, M - 1) * 4, 0);
@@ -186,13 +190,17 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
     // biases
     LDS_SPACE float* vectors = (LDS_SPACE float*)(lds + S::VECTORS_AT) + wave * 128;
     {
-        const int column = NB == 2 ? min(n_wave + (lane & 31), N - 1) : min(n_wave + lane, N - 1);
-        if constexpr (S::INT8) vectors[lane] = e.w_scale[NB == 2 && lane >= 32 ? N + column : column];
+        const int column = NB == 2 ? min(n_wave + lane % COLUMNS, N - 1) : min(n_wave + lane, N - 1);
+        if constexpr (S::INT8) vectors[lane] = e.w_scale[NB == 2 && lane >= COLUMNS ? N + column : column];
         if constexpr (S::BIAS) vectors[64 + lane] = (float)e.bias[column];
     }
 
     // a lane's operand read at step t: row l % 32, slot (2 t + l / 32) ^ (l % 16), i.e. this base with 32 t xored in
     const uint32_t operand = in_row * ROW_BYTES + 16 * (half ^ (lane & 15));
+    auto operand_at = [&](int t) {   // (a row of a power of two of bytes: one xor; else a chunk's low four bits by xor, the rest added)
+        if constexpr ((ROW_BYTES & (ROW_BYTES - 1)) == 0) return operand ^ (32 * t);
+        else return (operand ^ (32 * t & 255)) + (32 * t & ~255);
+    };
     const size_t row_bytes = (size_t)N * sizeof(OutT);
     // a lane's first 16-byte store (and residual load): row l % 32 of the block, columns n_wave + 8 (l / 32) ..; columns
     // past N store nothing (and load zeros)
@@ -217,19 +225,20 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
         const int col = 32 * (g / 4) + 8 * (g % 4) + 4 * half;
         Columns c{};
         if constexpr (S::INT8) c.scale = *(const LDS_SPACE v4f*)(vectors + col);
-        if constexpr (NB == 2) c.up = *(const LDS_SPACE v4f*)(vectors + 32 + col);
+        if constexpr (NB == 2) c.up = *(const LDS_SPACE v4f*)(vectors + COLUMNS + col);
         if constexpr (S::BIAS) c.bias = *(const LDS_SPACE v4f*)(vectors + 64 + col);
         return c;
     };
     // Output k of set D (fragment k / 16, register k % 16): lane l holds row l % 32 and, in register 4 q + r, column
-    // 8 q + 4 (l / 32) + r of its fragment
+    // 8 q + 4 (l / 32) + r of its fragment. Gated: up's sum is in the other fragment, or in the second half of the only one.
     auto output = [&](auto set, int k, const Columns& c) {
         constexpr int D = decltype(set)::value;
         const int f = k / 16, q = k % 16 / 4, r = k % 4;
+        constexpr int UP_FRAGMENT = FRAGMENTS - 1, UP_REGISTER = FRAGMENTS == 2 ? 0 : 8;
         float value;
         if constexpr (NB == 2 && !S::BIAS) {   // silu_times' constants on the row scale
             value = silu_times((MMA::value(sums[D][0], 4 * q + r) * (row_scale[D] * NEG_LOG2E)) * c.scale[r],
-                               (MMA::value(sums[D][1], 4 * q + r) * (row_scale[D] * NEG_LN2)) * c.up[r]);
+                               (MMA::value(sums[D][UP_FRAGMENT], UP_REGISTER + 4 * q + r) * (row_scale[D] * NEG_LN2)) * c.up[r]);
         } else {
             if constexpr (S::INT8) {
                 value = (MMA::value(sums[D][f], 4 * q + r) * row_scale[D]) * c.scale[r];
@@ -238,23 +247,42 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
             }
             if constexpr (S::BIAS) value = value + c.bias[r];
             if constexpr (NB == 2) {
-                const float up = (MMA::value(sums[D][1], 4 * q + r) * row_scale[D]) * c.up[r];
+                const float up = (MMA::value(sums[D][UP_FRAGMENT], UP_REGISTER + 4 * q + r) * row_scale[D]) * c.up[r];
                 value = silu_times(value * NEG_LOG2E, up * NEG_LN2);
             }
         }
         asm volatile("" : "+v"(value));   // the f32 value is what rounds
         return value;
     };
-    // the outputs of groups q = 2 p, 2 p + 1 of fragment f stored (plus the residual, its 8 columns in the lane's 16 bytes)
-    auto store = [&](const BufferResource& out_rsrc, int f, int p, const float (&even)[4], const float (&odd)[4], uint4 residual) {
+    // the residual's and the input's 8 columns of each of the lane's stores
+    struct Added { uint4 residual, original; };
+    constexpr int ADDED = S::RESIDUAL ? S::STORE_OPS : 1;
+    auto load_added = [&](int m0, Added (&added)[ADDED]) {
         if constexpr (S::RESIDUAL) {
-            float eight[8], lower[4], upper[4];
-            eight_values(even, odd, eight);
-            const v8h added = __builtin_bit_cast(v8h, residual);
+            const BufferResource residual_rsrc = rows_of(e.residual, m0);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                lower[j] = eight[j] + (float)added[j];
-                upper[j] = eight[4 + j] + (float)added[4 + j];
+            for (int j = 0; j < S::STORE_OPS; j++) added[j].residual = buffer_load16(residual_rsrc, at(j / 2, j % 2), 0);
+        }
+        if constexpr (S::MIX) {
+            const BufferResource original_rsrc = rows_of(e.original, m0);
+#pragma unroll
+            for (int j = 0; j < S::STORE_OPS; j++) added[j].original = buffer_load16(original_rsrc, at(j / 2, j % 2), 0);
+        }
+    };
+    const float mix_residual = S::MIX ? (float)e.residual_scale[0] : 0.0f, mix_input = S::MIX ? (float)e.input_scale[0] : 0.0f;
+    // the outputs of groups q = 2 p, 2 p + 1 of fragment f stored (plus the residual, its 8 columns in the lane's 16 bytes, and
+    // the next block's input mix)
+    auto store = [&](const BufferResource& out_rsrc, int f, int p, const float (&even)[4], const float (&odd)[4], const Added& more) {
+        if constexpr (S::RESIDUAL) {
+            float eight[8];
+            eight_values(even, odd, eight);
+            const v8h added = __builtin_bit_cast(v8h, more.residual), original = __builtin_bit_cast(v8h, more.original);
+            float lower[4], upper[4];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                float value = eight[j] + (float)added[j];
+                if constexpr (S::MIX) value = (to_float(from_float<OutT>(value)) * mix_residual) + ((float)original[j] * mix_input);
+                (j < 4 ? lower : upper)[j % 4] = value;
             }
             const uint2 lo = pack_four<OutT>(lower), hi = pack_four<OutT>(upper);
             buffer_store16(out_rsrc, v4u{lo.x, lo.y, hi.x, hi.y}, at(f, p), 0);
@@ -278,7 +306,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
     // group's column vectors read ahead into a slot of their own (read just before use, a vector's wait would also wait
     // for the operand reads ahead of it). The operand of step t + LOOKAHEAD is read at step t, and the DMA of block
     // b + STAGES - 1 goes out one instruction every DMA_EVERY steps.
-    constexpr int LOOKAHEAD = 2, DMA_EVERY = 3, PER_LANE = 16 * OUTPUTS, SPAN = 4 * STEPS / PER_LANE;   // a 4-column group's steps
+    constexpr int LOOKAHEAD = 2, DMA_EVERY = 3, PER_LANE = S::PER_LANE, SPAN = 4 * STEPS / PER_LANE;   // a 4-column group's steps
     static_assert(DMA_EVERY * (S::DMA_OPS - 1) < STEPS, "the turn's DMA fits its steps");
     auto turn = [&](auto set, int b, auto finishing) {
         constexpr int P = decltype(set)::value, D = 1 - P;
@@ -288,17 +316,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
         const LDS_SPACE int8_t* block = ring + stage * S::BLOCK_BYTES;
         const int m0 = (first + b - 1) * ROWS;   // the block before, whose epilogue this turn runs
         const BufferResource out_rsrc = rows_of(out, FINISH ? m0 : 0);
-        uint4 residual[S::RESIDUAL ? S::STORE_OPS : 1] = {};
-        if constexpr (S::RESIDUAL && FINISH) {
-            const BufferResource residual_rsrc = rows_of(e.residual, m0);
-#pragma unroll
-            for (int j = 0; j < S::STORE_OPS; j++) residual[j] = buffer_load16(residual_rsrc, at(j / 2, j % 2), 0);
-        }
+        Added added[ADDED] = {};
+        if constexpr (FINISH) load_added(m0, added);
         Columns slot[2];
         if constexpr (FINISH) slot[0] = columns(0);
         Operand a[STEPS];
 #pragma unroll
-        for (int t = 0; t < LOOKAHEAD; t++) a[t] = *(const LDS_SPACE Operand*)(block + (operand ^ (32 * t)));
+        for (int t = 0; t < LOOKAHEAD; t++) a[t] = *(const LDS_SPACE Operand*)(block + operand_at(t));
         float even[4], odd[4];
 #pragma unroll
         for (int t = 0; t < STEPS; t++) {
@@ -309,7 +333,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
                 for (int g = 1; g < PER_LANE / 4; g++)
                     if (t == g * SPAN - SPAN / 2) slot[g % 2] = columns(g);
             }
-            if (t + LOOKAHEAD < STEPS) a[t + LOOKAHEAD] = *(const LDS_SPACE Operand*)(block + (operand ^ (32 * (t + LOOKAHEAD))));
+            if (t + LOOKAHEAD < STEPS) a[t + LOOKAHEAD] = *(const LDS_SPACE Operand*)(block + operand_at(t + LOOKAHEAD));
 #pragma unroll
             for (int f = 0; f < FRAGMENTS; f++)
                 sums[P][f] = MMA::step(weights[f][t], a[t], t == 0 ? typename MMA::Sums{} : sums[P][f]);
@@ -319,7 +343,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
                 for (int k = t * PER_LANE / STEPS; k < (t + 1) * PER_LANE / STEPS; k++) {
                     const int q = k % 16 / 4, r = k % 4;
                     (q % 2 ? odd : even)[r] = output(std::integral_constant<int, D>{}, k, slot[k / 4 % 2]);
-                    if (q % 2 && r == 3) store(out_rsrc, k / 16, q / 2, even, odd, residual[S::RESIDUAL ? k / 16 * 2 + q / 2 : 0]);
+                    if (q % 2 && r == 3) store(out_rsrc, k / 16, q / 2, even, odd, added[S::RESIDUAL ? k / 16 * 2 + q / 2 : 0]);
                 }
             }
         }
@@ -330,18 +354,14 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
         constexpr int P = decltype(set)::value;
         const int m0 = (first + b) * ROWS;
         const BufferResource out_rsrc = rows_of(out, m0);
-        uint4 residual[S::RESIDUAL ? S::STORE_OPS : 1] = {};
-        if constexpr (S::RESIDUAL) {
-            const BufferResource residual_rsrc = rows_of(e.residual, m0);
-#pragma unroll
-            for (int j = 0; j < S::STORE_OPS; j++) residual[j] = buffer_load16(residual_rsrc, at(j / 2, j % 2), 0);
-        }
+        Added added[ADDED] = {};
+        load_added(m0, added);
         float even[4], odd[4];
 #pragma unroll
         for (int k = 0; k < PER_LANE; k++) {
             const int q = k % 16 / 4, r = k % 4;
             (q % 2 ? odd : even)[r] = output(std::integral_constant<int, P>{}, k, columns(k / 4));
-            if (q % 2 && r == 3) store(out_rsrc, k / 16, q / 2, even, odd, residual[S::RESIDUAL ? k / 16 * 2 + q / 2 : 0]);
+            if (q % 2 && r == 3) store(out_rsrc, k / 16, q / 2, even, odd, added[S::RESIDUAL ? k / 16 * 2 + q / 2 : 0]);
         }
     };
     if (idle) {
@@ -384,10 +404,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
 // The launch: a workgroup a compute unit, each XCD's workgroups taking streams of row blocks for every column group. A last
 // group with columns for only some wavefronts gets fewer workgroups and longer streams: its turns cost about
 // (WAVES + working wavefronts) / (2 WAVES) of a full group's.
-template <typename In, int NB, typename OutT, int EPI>
+template <typename In, int NB, typename OutT, int EPI, int DEPTH_ = DEPTH>
 int launch(const void* x, const void* w, void* out, const Epilogue& e, int M, int N, hipStream_t stream) {
-    typedef Shape<In, NB, EPI> S;
-    auto kernel = resident_kernel<In, NB, OutT, EPI>;
+    typedef Shape<In, NB, EPI, DEPTH_> S;
+    auto kernel = resident_kernel<In, NB, OutT, EPI, DEPTH_>;
     static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS_BYTES);
     if (allowed != hipSuccess) return (int)allowed;
     int device = 0, units = 0;
@@ -430,6 +450,71 @@ int dispatch(const void* x, const void* w, void* out, const Epilogue& e, int M, 
         return e.flags & EPI_RESIDUAL ? launch<In, 1, OutT, EPI_BIAS | EPI_RESIDUAL>(x, w, out, e, M, N, stream)
                                       : launch<In, 1, OutT, EPI_BIAS>(x, w, out, e, M, N, stream);
     }
+}
+
+// What tile 0 gives to this kernel: tile 15's launches and, with the same limits, the other depths of the networks' widths.
+// f(depth, epilogue), as constants, launches one; a launch that no instantiation takes is false.
+template <typename In, int NB, typename OutT, typename F> bool taken(int flags, int K, F&& f) {
+    constexpr bool INT8 = std::is_same<In, int8_t>::value;
+    auto with = [&](auto depth, auto epilogue) {
+        if (K != decltype(depth)::value || flags != decltype(epilogue)::value) return false;
+        f(depth, epilogue);
+        return true;
+    };
+    constexpr std::integral_constant<int, 0> PLAIN{};
+    constexpr std::integral_constant<int, EPI_BIAS> BIAS{};
+    constexpr std::integral_constant<int, EPI_RESIDUAL> RESIDUAL{};
+    constexpr std::integral_constant<int, EPI_RESIDUAL | EPI_MIX> MIX{};
+    constexpr std::integral_constant<int, EPI_BIAS | EPI_RESIDUAL> BIAS_RESIDUAL{};
+    constexpr std::integral_constant<int, 256> D256{};
+    constexpr std::integral_constant<int, 512> D512{};
+    constexpr std::integral_constant<int, 768> D768{};
+    constexpr std::integral_constant<int, 1024> D1024{};
+    if constexpr (sizeof(OutT) != 2 || (!INT8 && NB == 2)) {
+        return false;
+    } else if constexpr (!INT8) {
+        return with(D256, BIAS) || with(D256, BIAS_RESIDUAL) || with(D512, BIAS) || with(D512, BIAS_RESIDUAL);
+    } else if constexpr (NB == 2) {
+        return with(D256, PLAIN) || with(D512, PLAIN) || with(D768, PLAIN);
+    } else {
+        return with(D256, BIAS) || with(D512, BIAS) || with(D512, PLAIN) || with(D768, BIAS) || with(D1024, BIAS) || with(D1024, RESIDUAL)
+            || with(D1024, MIX);
+    }
+}
+
+// The least row blocks a workgroup's stream has to hold for the launch to pay for its weights' load and its ends. Timed on an
+// MI355X as graphs of launches (us, this kernel and the best other tile): int8, 768 to 1,152 columns, 17,920 rows (11 blocks)
+// 25.3 and 25.2, 35,000 40.7 and 44.3, 69,930 75.1 and 92.2; 768 to 2 x 992 gated, 7,000 (7) 19.8 and 17.2, 17,920 (17)
+// 35.5 and 38.3, 69,930 113 and 141; 256 to 2 x 1,024 gated, 17,920 (9) 21.5 and 20.0, 69,930 (34) 56.4 and 64.2; 256 to 832,
+// 17,920 (4) 14.9 and 11.7, 69,930 (17) 31.6 and 35.4; 1,024 to 768 with the residual and the mix, 17,920 (7) 29.4 and 32.2,
+// 35,000 (13) 46.8 and 54.4; 1,024 to 256 so, 35,000 (4) 25.7 and 25.0, 69,930 (9) 36.5 and 41.1; fp16, 256 to 256 with bias
+// and residual, 69,930 (9) 22.4 and 24.5. (Left out, as no faster: the residual at depths 512 and 768.) A launch of one output a
+// weight row that writes more than the last-level cache's 256 MB is bound by its writes, and whole lines from LDS go faster
+// than these 16-byte stores (512 to 2,048 at 65,536 rows, 268 MB: 121 us and 109 on tile 4; 512 to 1,600 at 71,680, 229 MB: 89
+// and 105); gated, 293 MB still take 163 and 240.
+constexpr int STREAM_BLOCKS = 10, DEEP_STREAM_BLOCKS = 6, F16_STREAM_BLOCKS = 8;
+constexpr uint64_t MOST_WRITTEN = 256ull << 20;
+
+template <typename In, int NB, typename OutT> bool takes(int flags, int M, int N, int K) {
+    if (N % 8 != 0 || (uint64_t)M * N * sizeof(OutT) >= (NB == 1 ? MOST_WRITTEN : 1ull << 31)) return false;
+    int device = 0, units = 0;
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return false;
+    bool worth = false;
+    const bool known = taken<In, NB, OutT>(flags, K, [&](auto depth, auto epilogue) {
+        typedef Shape<In, NB, decltype(epilogue)::value, decltype(depth)::value> S;
+        const int groups = (N + S::GROUP - 1) / S::GROUP;
+        const int least = !S::INT8 ? F16_STREAM_BLOCKS : S::RESIDUAL ? DEEP_STREAM_BLOCKS : STREAM_BLOCKS;
+        worth = groups <= units / XCDS && (long)(M / ROWS) * groups >= (long)least * units;
+    });
+    return known && worth;
+}
+template <typename In, int NB, typename OutT>
+int launch_taken(const void* x, const void* w, void* out, const Epilogue& e, int M, int N, int K, hipStream_t stream) {
+    int status = CHESS_OK;
+    taken<In, NB, OutT>(e.flags, K, [&](auto depth, auto epilogue) {
+        status = launch<In, NB, OutT, decltype(epilogue)::value, decltype(depth)::value>(x, w, out, e, M, N, stream);
+    });
+    return status;
 }
 
 }  // namespace resident

@@ -517,12 +517,12 @@ int by_tile(const void* x, const void* w, void* out, const Epilogue& e, int M, i
     }
 }
 
-// The tile for tile 0: int8 launches of 32,768 rows or more take the eight-wavefront 256 x 128; other large launches the
+// The tile for tile 0, where the register-held kernel does not take the launch (resident::takes): int8 launches of 32,768 rows or more take the eight-wavefront 256 x 128; other large launches the
 // 2-stage 128 x 128, with 128-byte stages for rows of 2 KB or more that are a multiple of 128 bytes (each L2 line of an
 // operand row read once); launches that still give the chip a 128 x 128 workgroup a compute unit take 128-byte stages
 // for any row of a multiple of 128 bytes, smaller ones the 128 x 64 tiles (128-byte stages where the rows allow), the
 // smallest 64 x 64. Timed on an MI355X (int8, bf16 out, bias, graphs of 30 launches): M = 65,536 by 512 -> 2,048 in
-// 124.7 against 127.6 us (tile 11), 2,048 -> 512 in 84.6 against 89.6 (tile 13), 512 -> 1,536 in 94.5 against 96.2;
+// 124.7 against 127.6 us (tile 11), 2,048 -> 512 in 84.6 against 89.6 (tile 13);
 // M = 16,384 by 512 -> 512 in 11.7 against 12.6 us and 2,048 -> 512 in 25.1 against 29.0 (tile 2); M = 4,096 by
 // 2,048 -> 512 in 10.3 against 10.5 (tile 3).
 template <typename In> int tile_by_size(int M, int N, int K) {
@@ -541,7 +541,10 @@ template <typename In> int tile_by_size(int M, int N, int K) {
 // rounded (half the LDS of the f32 staging).
 template <typename In, int NB, typename OutT>
 int dispatch(const void* x, const void* w, void* out, const Epilogue& e, int M, int N, int K, int tile, hipStream_t stream) {
-    if (tile == 0) tile = tile_by_size<In>(M, N, K);
+    if (tile == 0) {
+        if (resident::takes<In, NB, OutT>(e.flags, M, N, K)) return resident::launch_taken<In, NB, OutT>(x, w, out, e, M, N, K, stream);
+        tile = tile_by_size<In>(M, N, K);
+    }
     if (tile == DEEP) {
         if constexpr (std::is_same<In, int8_t>::value && NB == 1 && sizeof(OutT) == 2) return deep::dispatch<OutT>(x, w, out, e, M, N, K, stream);
         return chess_fail(CHESS_UNSUPPORTED, "tile %d takes int8 rows, not gated, to fp16 or bf16", DEEP);

@@ -446,6 +446,27 @@ def test_the_register_tile_at_the_batch_1024_rows(device):
         assert same_bits(launch_int8_linear(x, x_scale, weight, weight_scale, bias, residual, gated, *mix, int8_blocks.RESIDENT_TILE), expected)
 
 
+@pytest.mark.parametrize("matmul, depth, width", [("projection", 256, 520), ("projection", 512, 520), ("projection", 768, 1032),
+                                                  ("projection", 1024, 264), ("gate_up", 256, 264), ("gate_up", 768, 136),
+                                                  ("down", 1024, 264), ("mixing down", 1024, 264)])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16])
+def test_large_launches_of_tile_0_give_the_whole_k_tiles_bits(device, matmul, depth, width, out_dtype):
+    """Tile 0 holds the weights in registers where a workgroup's stream of row blocks is long: 41,007 rows (past each
+    epilogue's line; a ragged last block and a column group part past N) against tile 1, at every depth it has."""
+    x, x_scale, weight, weight_scale, bias, residual, gated, mix = int8_operands(matmul, 41007, device, width=width, depth=depth)
+    found = launch_int8_linear(x, x_scale, weight, weight_scale, bias, residual, gated, *mix, 0, out_dtype)
+    assert same_bits(found, launch_int8_linear(x, x_scale, weight, weight_scale, bias, residual, gated, *mix, 1, out_dtype))
+
+
+@pytest.mark.parametrize("depth", [256, 512])
+@pytest.mark.parametrize("with_residual", [True, False])
+def test_large_launches_of_tile_0_give_fp16_sums_the_whole_k_tiles_bits(device, depth, with_residual):
+    x, weight, bias, residual = output_projection_operands(41007, 264, device)
+    x, weight, residual = x[:, :depth].contiguous(), weight[:depth].contiguous(), residual if with_residual else None
+    found = launch_linear(x, weight, bias, residual, False, False, None, None, None, 0)
+    assert same_bits(found, launch_linear(x, weight, bias, residual, False, False, None, None, None, 1))
+
+
 def test_the_register_tile_refuses_what_it_cannot_take(device):
     """Tile 15 holds depth 512 in registers, stores 4 columns a lane and adds no residual or input mix: other depths,
     widths not a multiple of 8 and the down epilogues are refused."""
