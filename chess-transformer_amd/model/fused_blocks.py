@@ -35,14 +35,23 @@ LINEAR_TILES = {"gfx950": [(5, 1), (9, 3), (48, 6), (100, 11), (math.inf, 15)]}
 # projection to 1,600 columns: 155.7 against 200.2 us on tile 0); other linears of the table's share take tile 0, the
 # kernel's own pick by size
 RESIDENT_TILE, RESIDENT_DEPTH = 15, 512
+# and from this share on where it has 1,024 columns or more, so that each of its workgroups still has a long stream of row
+# blocks (512 to 1,600 columns at 17,920 rows, graphs of launches: 37.4 against 43.0 us on tile 11); up to 4,096, inside the
+# column groups and output bytes it takes
+RESIDENT_WIDE_SHARE, RESIDENT_WIDE_COLUMNS = 48, range(1024, 4097)
+# gated: at 512 to 2 x 2,048 (graphs of launches, us) 4,480 rows take 27.0 on tile 12 and 29.6 on tile 6, 35,840 rows 172.8 on
+# the eight-wavefront 256 x 128 tile 4 and 175.6 on tile 11, 71,680 rows 333 and 336; 768 to 2 x 992 at 49,000 rows 167 and 181
+LINEAR_GATED_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (100, 11), (math.inf, 4)]}
 # f32 out (accumulate_fp32, the policy head's `a`): its f32 staging runs faster at 128 x 128 with a 3-stage ring (78 against
 # 97 us at 71,680 rows on an MI355X)
 LINEAR_F32_TILES = {"gfx950": [(4, 1), (math.inf, 7)]}
-# rows of 2 KB or more (the fp16 block's down, 2,048 inputs), not gated: 128 x 128 with 128-byte stages, whole L2 lines a
-# step (190 against 226 us at 71,680 rows); 128 x 64 with 128-byte stages up to 160 rows a compute unit (batch 64 / 256:
-# 22.0 / 57.6 against 23.8 / 58.0 us) and 64 x 64 up to 9 (batch 16: 11.8 against 20.7 us)
-LINEAR_LONG_ROW_TILES = {"gfx950": [(9, 1), (160, 12), (math.inf, 13)]}
-LONG_ROW_BYTES = 2048
+# rows of 1.5 KB or more (the fp16 block's down, combine of a width of 768 or more), not gated: 128 x 128 with 128-byte stages,
+# whole L2 lines a step (2,048 inputs: 190 against 226 us at 71,680 rows, 94 against 101 with tile 12 at 35,840; 768 inputs to
+# 768: 79.2 against 91.9 with tile 11 at 49,000); 128 x 64 with 128-byte stages up to 100 rows a compute unit (2,048 inputs at
+# 17,920 rows 54.7 against 58.2 us, 768 inputs 36.8 against 38.6 with tile 11; batch 64 22.0 against 23.8) and 64 x 64 up to 9
+# (batch 16: 11.8 against 20.7 us)
+LINEAR_LONG_ROW_TILES = {"gfx950": [(9, 1), (100, 12), (math.inf, 13)]}
+LONG_ROW_BYTES = 1536
 # from this many (position, key/value group) pairs groups_per_workgroup plans a launch of 65 to 80 tokens, query and value
 # widths up to 64, for workgroups of four wavefronts instead of five. (Such launches, and those of 64 tokens, share their pairs
 # out by themselves and only check that the run divides them: csrc/attention_wave.h.)
@@ -65,7 +74,9 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
     arch = torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
     if accumulate_fp32:
         table = LINEAR_F32_TILES
-    elif row_bytes >= LONG_ROW_BYTES and row_bytes % 128 == 0 and not gated:
+    elif gated:
+        table = LINEAR_GATED_TILES
+    elif row_bytes >= LONG_ROW_BYTES and row_bytes % 128 == 0:
         table = LINEAR_LONG_ROW_TILES
     else:
         table = LINEAR_TILES
@@ -217,8 +228,12 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
            gated: bool = False, accumulate_fp32: bool = False, original: torch.Tensor | None = None, residual_scale: torch.Tensor | None = None,
            input_scale: torch.Tensor | None = None) -> torch.Tensor:
     K, width = weight.shape
-    tile = linear_tile(x.device, x.numel() // K, accumulate_fp32, K * x.element_size(), gated)
-    if not linear_takes(tile, K, width // 2 if gated else width, gated, bias is not None, residual is not None, accumulate_fp32, original is not None):
+    M, N = x.numel() // K, width // 2 if gated else width
+    tile = linear_tile(x.device, M, accumulate_fp32, K * x.element_size(), gated)
+    takes = lambda tile: linear_takes(tile, K, N, gated, bias is not None, residual is not None, accumulate_fp32, original is not None)
+    if N in RESIDENT_WIDE_COLUMNS and M > RESIDENT_WIDE_SHARE * torch.cuda.get_device_properties(x.device).multi_processor_count and takes(RESIDENT_TILE):
+        tile = RESIDENT_TILE
+    elif not takes(tile):
         tile = 0
     return launch_linear(x, weight, bias, residual, gated, accumulate_fp32, original, residual_scale, input_scale, tile)
 
