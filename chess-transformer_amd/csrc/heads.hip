@@ -13,7 +13,7 @@
 // still spreads over the chip. Its wavefronts split D in up to 4 parts, whose partial blocks meet in LDS and are added in
 // part order. A step covers 8 of D: lane l (row l % 32, half h = l / 32) loads 4 consecutive values k0 + 4h .. + 3 of its
 // row of each operand and feeds them to 4 MFMAs, value m to MFMA m, so that in MFMA m both operands' k-halves stand for
-// k0 + m and k0 + 4 + m; eight steps' loads go out together. The blocks go to a workspace of the caller's, 7,168 floats a
+// k0 + m and k0 + 4 + m; four steps' loads go out together. The blocks go to a workspace of the caller's, 7,168 floats a
 // position (the 64 x 64 logits, then 96 x 32 narrow products). The second launch, a workgroup a position, adds each
 // square's narrow column 0, gathers the 1,968 moves with their promotion logits, and writes board_down's inputs.
 #include "chess_common.h"
@@ -36,30 +36,28 @@ DEVICE float gelu(float v) { return 0.5f * v * (1.0f + erff(v * 0.70710678118654
 
 // the 32 x 32 block sum_k A[row0 + i][k] * X[col0 + j][k] over k < length, rows stride elements apart: A's rows f32 (a_bias
 // added when BIAS), X's fp16; rows past a_rows and columns past x_rows read the last one (never kept). Lane l holds, in
-// register 4q + r, the sum for A row 8q + 4(l / 32) + r and X row l % 32. length is a multiple of 64: eight steps a turn,
-// their loads issued before their MFMAs, so that a turn's loads are in flight together.
+// register 4q + r, the sum for A row 8q + 4(l / 32) + r and X row l % 32. length is a multiple of 64: four steps a turn,
+// their loads (the bias's too) issued before their MFMAs, so that a turn's loads are in flight together.
 template <bool BIAS>
 DEVICE v16f block_products(const float* A, int a_rows, const float* a_bias, const half_t* X, int x_rows, int length, int stride, int lane) {
-    constexpr int TURN = 8;   // steps of 8 a turn
+    constexpr int TURN = 4;   // steps of 8 a turn
     const int r32 = lane & 31, h = lane >> 5;
     const float* a_row = A + (size_t)min(r32, a_rows - 1) * stride + 4 * h;
     const half_t* x_row = X + (size_t)min(r32, x_rows - 1) * stride + 4 * h;
     v16f acc = {};
     for (int turn = 0; turn < length; turn += 8 * TURN) {
-        float4 av[TURN];
+        float4 av[TURN], bias[TURN];
         v4h xv[TURN];
 #pragma unroll
         for (int s = 0; s < TURN; s++) {
             av[s] = *reinterpret_cast<const float4*>(a_row + turn + 8 * s);
             xv[s] = *reinterpret_cast<const v4h*>(x_row + turn + 8 * s);
+            if constexpr (BIAS) bias[s] = *reinterpret_cast<const float4*>(a_bias + turn + 8 * s + 4 * h);
         }
 #pragma unroll
         for (int s = 0; s < TURN; s++) {
             float4 a4 = av[s];
-            if constexpr (BIAS) {
-                const float4 bias = *reinterpret_cast<const float4*>(a_bias + turn + 8 * s + 4 * h);
-                a4 = float4{a4.x + bias.x, a4.y + bias.y, a4.z + bias.z, a4.w + bias.w};
-            }
+            if constexpr (BIAS) a4 = float4{a4.x + bias[s].x, a4.y + bias[s].y, a4.z + bias[s].z, a4.w + bias[s].w};
             acc = mfma_f32(a4.x, (float)xv[s][0], acc);
             acc = mfma_f32(a4.y, (float)xv[s][1], acc);
             acc = mfma_f32(a4.z, (float)xv[s][2], acc);
@@ -117,6 +115,12 @@ __global__ __launch_bounds__(THREADS) void head_blocks_kernel(
     }
 }
 
+// The moves and the values a thread takes in one turn, each kind of load issued for all of them before any is used: the chain
+// from a move's cells to its products is two trips long, and a loop over single moves paid it for each left over from its
+// unrolling. With the bias's loads above, on an MI355X at 512 columns: both launches at one position 14.4 -> 11.4 us, at 64
+// 19.5 -> 16.1, at 300 49.9 -> 46.8.
+constexpr int GATHER_TURN = 8, DOWN_TURN = 5;
+
 __global__ __launch_bounds__(THREADS) void head_gather_kernel(
     const float* __restrict__ workspace, const int* __restrict__ cells, const int* __restrict__ promotions, float* __restrict__ out,
     float* __restrict__ down, int T, int NN, int down_first, int moves, int out_stride, int activate)
@@ -129,19 +133,41 @@ __global__ __launch_bounds__(THREADS) void head_gather_kernel(
     // are masked into the blocks, so that no table entry reads outside them); logits = the quadrant + s[from] (the from
     // square's narrow column 0)
     float* out_b = out + b * out_stride;
-#pragma unroll 4
-    for (int m = tid; m < moves; m += THREADS) {
-        const int cell = cells[m], promotion = promotions[m], from = (cell >> 6) & 63;
-        float value = logits[from * SQUARES + (cell & 63)] + narrow[from * MAX_NARROW];
-        if (promotion >= 0) value = value + narrow[((promotion >> 5) & 63) * MAX_NARROW + (promotion & 31)];
-        out_b[m] = value;
+    for (int m0 = tid; m0 < moves; m0 += GATHER_TURN * THREADS) {
+        int cell[GATHER_TURN], promotion[GATHER_TURN];
+        float value[GATHER_TURN], s[GATHER_TURN], promoted[GATHER_TURN];
+#pragma unroll
+        for (int i = 0; i < GATHER_TURN; i++) {   // (a move past the last reads the last one's and is not written)
+            const int m = min(m0 + i * THREADS, moves - 1);
+            cell[i] = cells[m];
+            promotion[i] = promotions[m];
+        }
+#pragma unroll
+        for (int i = 0; i < GATHER_TURN; i++) {
+            const int from = (cell[i] >> 6) & 63;
+            value[i] = logits[from * SQUARES + (cell[i] & 63)];
+            s[i] = narrow[from * MAX_NARROW];
+            promoted[i] = promotion[i] >= 0 ? narrow[((promotion[i] >> 5) & 63) * MAX_NARROW + (promotion[i] & 31)] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < GATHER_TURN; i++) {
+            float sum = value[i] + s[i];
+            if (promotion[i] >= 0) sum = sum + promoted[i];
+            if (m0 + i * THREADS < moves) out_b[m0 + i * THREADS] = sum;
+        }
     }
-    const int width = NN - down_first;
-    float* down_b = down + b * T * width;
-#pragma unroll 4
-    for (int e = tid; e < T * width; e += THREADS) {
-        const float value = narrow[(e / width) * MAX_NARROW + down_first + e % width];
-        down_b[e] = activate ? gelu(value) : value;
+    const int width = NN - down_first, values = T * width;
+    float* down_b = down + b * values;
+    for (int e0 = tid; e0 < values; e0 += DOWN_TURN * THREADS) {
+        float value[DOWN_TURN];
+#pragma unroll
+        for (int i = 0; i < DOWN_TURN; i++) {
+            const int e = min(e0 + i * THREADS, values - 1), token = e / width;
+            value[i] = narrow[token * MAX_NARROW + down_first + e - token * width];
+        }
+#pragma unroll
+        for (int i = 0; i < DOWN_TURN; i++)
+            if (e0 + i * THREADS < values) down_b[e0 + i * THREADS] = activate ? gelu(value[i]) : value[i];
     }
 }
 
@@ -161,6 +187,10 @@ constexpr int MAX_BINS = 128;
 // take the K chunks in turn (wavefront w the chunks w, w + 4, ...), and their partial tiles are added in LDS as
 // (w0 + w1) + (w2 + w3): a fixed order, so that no position's units depend on the batch it is in. Lane l ends with
 // positions 4 (l / 16) + r (register r) of unit l % 16.
+// A wavefront's chunks go in turns of HIDDEN_TURN, a turn's loads all in flight together, the last turn's missing chunks left
+// out by a branch the whole wavefront takes (17 of the 70 chunks in a loop unrolled by 6 left 5 to go one by one).
+constexpr int HIDDEN_TURN = 6;
+
 __global__ __launch_bounds__(THREADS) void value_hidden_kernel(const float* __restrict__ c, const float* __restrict__ weight,
                                                                const float* __restrict__ bias, float* __restrict__ hidden, int B, int K, int H)
 {
@@ -171,14 +201,24 @@ __global__ __launch_bounds__(THREADS) void value_hidden_kernel(const float* __re
     const float* a_row = c + (size_t)min(p0 + row, B - 1) * K + 4 * group;
     const float* b_row = weight + (size_t)(u0 + row) * K + 4 * group;
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 6
-    for (int chunk = wave; chunk < K / VALUE_CHUNK; chunk += 4) {
-        const float4 a4 = *reinterpret_cast<const float4*>(a_row + chunk * VALUE_CHUNK);
-        const float4 b4 = *reinterpret_cast<const float4*>(b_row + chunk * VALUE_CHUNK);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.x, b4.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.y, b4.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.z, b4.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.w, b4.w, acc, 0, 0, 0);
+    const int chunks = K / VALUE_CHUNK;
+    for (int first = wave; first < chunks; first += 4 * HIDDEN_TURN) {   // (a chunk past K reads the last one and is left out)
+        float4 a4[HIDDEN_TURN], b4[HIDDEN_TURN];
+#pragma unroll
+        for (int i = 0; i < HIDDEN_TURN; i++) {
+            const int chunk = min(first + 4 * i, chunks - 1);
+            a4[i] = *reinterpret_cast<const float4*>(a_row + chunk * VALUE_CHUNK);
+            b4[i] = *reinterpret_cast<const float4*>(b_row + chunk * VALUE_CHUNK);
+        }
+#pragma unroll
+        for (int i = 0; i < HIDDEN_TURN; i++) {
+            if (first + 4 * i < chunks) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[i].x, b4[i].x, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[i].y, b4[i].y, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[i].z, b4[i].z, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[i].w, b4[i].w, acc, 0, 0, 0);
+            }
+        }
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) partial[wave][(4 * group + r) * VALUE_TILE + row] = acc[r];
@@ -189,11 +229,16 @@ __global__ __launch_bounds__(THREADS) void value_hidden_kernel(const float* __re
 }
 
 // The second layer, the softmax and the expected score, a workgroup a position: thread t takes bin t % 128 over half t / 128
-// of the units (its W2 row read 16 bytes at a time, the position's hidden row uniform across each wavefront), f32 fma along
+// of the units (its W2 row from LDS, the position's hidden row uniform across each wavefront), f32 fma along
 // its units in order; the halves meet in LDS as first + second, then wavefront 0 holds bins l and l + 64 in lane l and takes
 // the maximum, the exponentials' sum and the centres' weighted sum as wavefront trees. A position's chain of dependent
 // loads is a quarter of one wavefront's walk over all the units, and a batch of few positions still spreads over the chip.
+// W2 comes through LDS, in rows of 64 units that 16 lanes read as two whole lines: read straight into the lanes that sum it, each
+// 16-byte load touched 64 lines. Both launches of the value head, on an MI355X at 512 units and 81 bins: one position 14.9 ->
+// 13.4 us, 300 31.2 -> 26.6, 1,024 64.3 -> 55.6.
 constexpr int SCORE_PARTS = THREADS / MAX_BINS;
+constexpr int SCORE_UNITS = 64;                   // units of a part staged at a time
+constexpr int SCORE_ROW = SCORE_UNITS + 4;        // and a row's floats in LDS: 64 lanes' 16-byte reads fall in all banks
 
 __global__ __launch_bounds__(THREADS) void value_score_kernel(const float* __restrict__ hidden, const float* __restrict__ weight,
                                                               const float* __restrict__ bias, const float* __restrict__ centres,
@@ -201,17 +246,44 @@ __global__ __launch_bounds__(THREADS) void value_score_kernel(const float* __res
                                                               int row_stride, int score_column)
 {
     __shared__ float partial[SCORE_PARTS][MAX_BINS];
+    __shared__ __align__(16) float staged[SCORE_PARTS * MAX_BINS * SCORE_ROW];
+    __shared__ __align__(16) float staged_hidden[SCORE_PARTS * SCORE_UNITS];
     const int tid = threadIdx.x, lane = tid & 63;
     const int b = blockIdx.x;
-    const int v = tid % MAX_BINS, part = tid / MAX_BINS, units = H / SCORE_PARTS;
-    const float* h = hidden + (size_t)b * H + part * units;
-    const float* wv = weight + (size_t)min(v, bins - 1) * H + part * units;
+    const int v = tid % MAX_BINS, part = __builtin_amdgcn_readfirstlane(tid / MAX_BINS), units = H / SCORE_PARTS;
+    // staging item i of a thread: 16 bytes of a bin's row (the last bin's again past it), and of the hidden row; the next
+    // units' items are in flight while these are summed
+    constexpr int QUARTS = SCORE_UNITS / 4, ITEMS = SCORE_PARTS * MAX_BINS * QUARTS / THREADS;
+    v4f next[ITEMS], next_hidden;
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) {
+            const int item = tid + i * THREADS, to = item / QUARTS, k = min(k0 + item % QUARTS * 4, units - 4);
+            next[i] = *reinterpret_cast<const v4f*>(weight + (size_t)min(to / SCORE_PARTS, bins - 1) * H + to % SCORE_PARTS * units + k);
+        }
+        next_hidden = *reinterpret_cast<const v4f*>(hidden + (size_t)b * H + tid / QUARTS % SCORE_PARTS * units + min(k0 + tid % QUARTS * 4, units - 4));
+    };
     float sum = 0.0f;
+    load(0);
+    for (int k0 = 0; k0 < units; k0 += SCORE_UNITS) {
+        if (k0 > 0) __syncthreads();   // the units before are summed
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) {
+            const int item = tid + i * THREADS, to = item / QUARTS;
+            *reinterpret_cast<v4f*>(staged + (to % SCORE_PARTS * MAX_BINS + to / SCORE_PARTS) * SCORE_ROW + item % QUARTS * 4) = next[i];
+        }
+        if (tid < SCORE_PARTS * QUARTS) reinterpret_cast<v4f*>(staged_hidden)[tid] = next_hidden;
+        __syncthreads();
+        load(min(k0 + SCORE_UNITS, units - 4));   // (past the last: the same place again, not used)
+        const float* row = staged + (part * MAX_BINS + v) * SCORE_ROW;
+        const float* h = staged_hidden + part * SCORE_UNITS;
+        const int here = min(SCORE_UNITS, units - k0);
 #pragma unroll 8
-    for (int k = 0; k < units; k += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(h + k);
-        const float4 a = *reinterpret_cast<const float4*>(wv + k);
-        sum = __builtin_fmaf(x.x, a.x, sum); sum = __builtin_fmaf(x.y, a.y, sum); sum = __builtin_fmaf(x.z, a.z, sum); sum = __builtin_fmaf(x.w, a.w, sum);
+        for (int k = 0; k < here; k += 4) {
+            const v4f x = *reinterpret_cast<const v4f*>(h + k);
+            const v4f a = *reinterpret_cast<const v4f*>(row + k);
+            sum = __builtin_fmaf(x[0], a[0], sum); sum = __builtin_fmaf(x[1], a[1], sum); sum = __builtin_fmaf(x[2], a[2], sum); sum = __builtin_fmaf(x[3], a[3], sum);
+        }
     }
     partial[part][v] = sum;
     __syncthreads();

@@ -42,9 +42,12 @@ RESIDENT_WIDE_SHARE, RESIDENT_WIDE_COLUMNS = 48, range(1024, 4097)
 # gated: at 512 to 2 x 2,048 (graphs of launches, us) 4,480 rows take 27.0 on tile 12 and 29.6 on tile 6, 35,840 rows 172.8 on
 # the eight-wavefront 256 x 128 tile 4 and 175.6 on tile 11, 71,680 rows 333 and 336; 768 to 2 x 992 at 49,000 rows 167 and 181
 LINEAR_GATED_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (100, 11), (math.inf, 4)]}
-# f32 out (accumulate_fp32, the policy head's `a`): its f32 staging runs faster at 128 x 128 with a 3-stage ring (78 against
-# 97 us at 71,680 rows on an MI355X)
-LINEAR_F32_TILES = {"gfx950": [(4, 1), (math.inf, 7)]}
+# f32 out (accumulate_fp32, the policy head's `a`), graphs of launches on an MI355X, us: rows shorter than LONG_ROW_BYTES and of
+# whole lines take 128 x 64 with 128-byte stages (512 to 512: 9.2 against 10.5 on tile 7 at 4,480 rows, 25.0 against 32.1 at
+# 17,920, 78.6 against 83.7 at 71,680) and 64 x 64 up to 9 rows a compute unit (1,120 rows 5.6 against 9.4); longer ones the
+# 128 x 128 with a 3-stage ring (768 to 768 at 21,000 rows: 53.6 against 57.1)
+LINEAR_F32_TILES = {"gfx950": [(9, 1), (math.inf, 12)]}
+LINEAR_F32_LONG_ROW_TILES = {"gfx950": [(4, 1), (math.inf, 7)]}
 # rows of 1.5 KB or more (the fp16 block's down, combine of a width of 768 or more), not gated: 128 x 128 with 128-byte stages,
 # whole L2 lines a step (2,048 inputs: 190 against 226 us at 71,680 rows, 94 against 101 with tile 12 at 35,840; 768 inputs to
 # 768: 79.2 against 91.9 with tile 11 at 49,000); 128 x 64 with 128-byte stages up to 100 rows a compute unit (2,048 inputs at
@@ -73,7 +76,7 @@ def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: b
 def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False) -> int:
     arch = torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
     if accumulate_fp32:
-        table = LINEAR_F32_TILES
+        table = LINEAR_F32_TILES if row_bytes % 128 == 0 and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
     elif gated:
         table = LINEAR_GATED_TILES
     elif row_bytes >= LONG_ROW_BYTES and row_bytes % 128 == 0:
