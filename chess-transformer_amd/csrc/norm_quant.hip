@@ -90,7 +90,8 @@ template <int C, int LANES, bool VECTOR, bool FULL, typename T> DEVICE void stor
 // 1 / sqrt(tree_sum(v * v) / D + eps) of the group's row
 template <int C, int LANES> DEVICE float row_inverse(const float (&v)[C], int D, float eps) {
     typedef Split<C, LANES> S;
-    float partial[S::J];
+    constexpr int PLACES = S::J <= 2 ? S::J : S::J <= 4 ? 4 : 8;   // the tree's: chunks past J hold the padding's zeros
+    float partial[PLACES] = {};
 #pragma unroll
     for (int j = 0; j < S::J; j++) {
         float squares[S::W];
@@ -103,7 +104,7 @@ template <int C, int LANES> DEVICE float row_inverse(const float (&v)[C], int D,
         partial[j] = group_sum<LANES>(squares[0]);
     }
 #pragma unroll
-    for (int width = S::J; width > 1; width >>= 1)
+    for (int width = PLACES; width > 1; width >>= 1)
 #pragma unroll
         for (int i = 0; i < width / 2; i++) partial[i] = partial[2 * i] + partial[2 * i + 1];
     return 1.0f / __builtin_sqrtf(partial[0] / (float)D + eps);
@@ -224,15 +225,26 @@ int launch(const void* x, const void* original, const void* residual_scale, cons
     return launch_status();
 }
 
+// Rows of three quarters of a power of two (1,536, 768, and 384 in large launches) take 64, 32 or 16 lanes of 24 elements: full
+// rows, no masks and no lanes on the padding (rows of 768 took a whole wavefront padded to 1,024 columns, whose second half
+// of lanes held nothing in their second chunk; norm_quant on an MI355X, us: 49,000 rows 29.3 -> 19.5, 17,920 18.9 -> 9.5,
+// 3,570 5.8 -> 3.5, 70 3.0 -> 2.5; with the mix 46.8 -> 41.3, 23.0 -> 16.4, 7.6 -> 5.0, 3.5 -> 3.1; 16 lanes of 48 elements
+// 19.6 and 41.1 at 49,000 rows, 3.1 and 4.1 at 70). Others:
 // rows up to 512 (zero-padded to a power of two) in launches of GROUPED_ROWS or more take groups of 16 lanes, 4 to 32
 // elements a lane; else a whole wavefront a row, 1 to 32 elements a lane. Any split gives the same bits.
 template <bool QUANT>
 int by_width(const void* x, const void* original, const void* residual_scale, const void* input_scale, const void* gain, void* mixed, void* q,
              void* scale, void* normed, int M, int D, float eps, hipStream_t s)
 {
+    const bool grouped = M >= GROUPED_ROWS;
+    if (aligned16(gain) && D % 24 == 0) {   // three chunks a lane, exactly
+        if (D / 24 == 64) return launch<24, 64, QUANT>(x, original, residual_scale, input_scale, gain, mixed, q, scale, normed, M, D, eps, s);
+        if (D / 24 == 32) return launch<24, 32, QUANT>(x, original, residual_scale, input_scale, gain, mixed, q, scale, normed, M, D, eps, s);
+        if (D / 24 == 16 && grouped)
+            return launch<24, 16, QUANT>(x, original, residual_scale, input_scale, gain, mixed, q, scale, normed, M, D, eps, s);
+    }
     int padded = 64;
     while (padded < D) padded <<= 1;
-    const bool grouped = M >= GROUPED_ROWS;
     switch (padded) {
         case 64: return grouped ? launch<4, 16, QUANT>(x, original, residual_scale, input_scale, gain, mixed, q, scale, normed, M, D, eps, s)
                                 : launch<1, 64, QUANT>(x, original, residual_scale, input_scale, gain, mixed, q, scale, normed, M, D, eps, s);

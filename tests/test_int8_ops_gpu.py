@@ -95,6 +95,23 @@ def test_norm_quant_of_large_launches_matches_the_oracle_to_the_bit(device, rows
     assert bits_equal(q, expected_q) and bits_equal(scale, expected_scale)
 
 
+@pytest.mark.parametrize("rows, D", [(1, 768), (31, 768), (33, 384), (16389, 384), (33, 1536), (32769, 1536), (33000, 776)])
+def test_norms_of_three_quarter_widths_match_the_oracle_to_the_bit(device, rows, D):
+    """Rows of 24 elements a lane, 16 (from 16,384 rows), 32 or 64 lanes to a row, with the ends of a wavefront's rows; and 776
+    columns, masked, two rows a whole wavefront from 32,768 rows."""
+    generator = torch.Generator(device="cpu").manual_seed(rows + D)
+    x = (torch.randn(rows, D, generator=generator) * 4).half()
+    original = torch.randn(rows, D, generator=generator).half()
+    gain = (torch.rand(D, generator=generator) + 0.5).half()
+    rs, is_ = torch.tensor([0.8]).half(), torch.tensor([0.5]).half()
+    on_device = [t.to(device) for t in (x, original, rs, is_, gain)]
+    for found, expected in zip(mix_norm_quant(*on_device, 1e-5), oracle.mix_norm_quant(*(t.numpy() for t in (x, original, rs, is_, gain)), 1e-5)):
+        assert bits_equal(found, expected)
+    for found, expected in zip(norm_quant(on_device[0], on_device[-1], 1e-5), oracle.norm_quant(x.numpy(), gain.numpy(), 1e-5)):
+        assert bits_equal(found, expected)
+    assert bits_equal(rms_norm(on_device[0], on_device[-1], 1e-5), oracle.rms_norm(x.numpy(), gain.numpy(), 1e-5)[1])
+
+
 def test_empty_batches_give_outputs_of_no_rows(device):
     """No positions: every operator on the path returns outputs of no rows and the right types (the C ABI launches nothing
     for them), the int8 GEMM on the table's tiles and on the register-held ones."""
