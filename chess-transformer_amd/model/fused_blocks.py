@@ -19,7 +19,7 @@ from torch import nn
 
 from model import hip_kernels
 from model.encoding import NUM_SQUARES, TOKENS_PER_BOARD
-from model.hip_kernels import aligned, check, library_for, pointer, stream_of
+from model.hip_kernels import aligned, check, gpu, library_for, pointer, stream_of
 from model.model import EDGE, KING, KNIGHT, NO_PIECE, PAWN, QUEEN, THEIRS, ChessTransformer, TransformerBlock, value_bin_centres
 
 LINEAR_DEPTH, GROUP_M = 32, 8
@@ -74,7 +74,7 @@ def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: b
 
 
 def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False) -> int:
-    arch = torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
+    arch, units = gpu(device)
     if accumulate_fp32:
         table = LINEAR_F32_TILES if row_bytes % 128 == 0 and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
     elif gated:
@@ -83,7 +83,7 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
         table = LINEAR_LONG_ROW_TILES
     else:
         table = LINEAR_TILES
-    return tile_for(table.get(arch, table["gfx950"]), M, torch.cuda.get_device_properties(device).multi_processor_count)
+    return tile_for(table.get(arch, table["gfx950"]), M, units)
 
 
 def attention_waves(positions: int, kv_heads: int, tokens: int, dq: int, dv: int) -> int:
@@ -127,7 +127,7 @@ def launch_template_attention(projected: torch.Tensor, templates: torch.Tensor, 
     projected = aligned(projected)
     keyed = keyed_templates(templates, templates_count)
     out = torch.empty(B, T, heads * dv, device=projected.device, dtype=projected.dtype)
-    groups = groups_per_block or groups_per_workgroup(B, kv_heads, torch.cuda.get_device_properties(projected.device).multi_processor_count, T, dq, dv)
+    groups = groups_per_block or groups_per_workgroup(B, kv_heads, gpu(projected.device)[1], T, dq, dv)
     entry = library.chess_template_attention_bf16 if bf16 else library.chess_template_attention
     code = entry(pointer(projected), pointer(keyed), pointer(q_gain.contiguous()), pointer(k_gain.contiguous()), pointer(out), B, T, heads,
                  kv_heads, dq, dv, templates_count, groups, float(eps), 1 / math.sqrt(dq), stream_of(projected.device))
@@ -234,7 +234,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     M, N = x.numel() // K, width // 2 if gated else width
     tile = linear_tile(x.device, M, accumulate_fp32, K * x.element_size(), gated)
     takes = lambda tile: linear_takes(tile, K, N, gated, bias is not None, residual is not None, accumulate_fp32, original is not None)
-    if N in RESIDENT_WIDE_COLUMNS and M > RESIDENT_WIDE_SHARE * torch.cuda.get_device_properties(x.device).multi_processor_count and takes(RESIDENT_TILE):
+    if N in RESIDENT_WIDE_COLUMNS and M > RESIDENT_WIDE_SHARE * gpu(x.device)[1] and takes(RESIDENT_TILE):
         tile = RESIDENT_TILE
     elif not takes(tile):
         tile = 0

@@ -87,6 +87,20 @@ def library_for(device: torch.device) -> ctypes.CDLL:
     return library
 
 
+# each GPU's target and compute units, by its index: they stand while the process runs, and torch builds a new object of all the
+# properties whenever it is asked, which the operators' choices of tiles did two or three times a call
+_gpus: dict[int, tuple[str, int]] = {}
+
+
+def gpu(device: torch.device) -> tuple[str, int]:
+    """The device's target (gfx950) and its compute units."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    if index not in _gpus:
+        properties = torch.cuda.get_device_properties(index)
+        _gpus[index] = properties.gcnArchName.split(":")[0], properties.multi_processor_count
+    return _gpus[index]
+
+
 def check(code: int, what: str) -> None:
     if code == 0:
         return

@@ -140,10 +140,11 @@ def int8_tile(device: torch.device, matmul: str, M: int, N: int = 0, K: int = 0,
     the table's entry for the rows a compute unit's share is, or, given N and K, the first entry from there on whose tile
     takes them with that epilogue (gated and residual default to the role's: gate_up gated, down with the residual; none
     takes them: 0, the kernel's own pick of a whole-K tile, which takes every shape)."""
-    tiles = INT8_TILES.get(gpu_arch(device), INT8_TILES["gfx950"])[matmul]
+    arch, units = hip_kernels.gpu(device)
+    tiles = INT8_TILES.get(arch, INT8_TILES["gfx950"])[matmul]
     if matmul == "projection" and K > RESIDENT_DEPTH and K % 128 == 0:
-        tiles = LONG_PROJECTION_TILES.get(gpu_arch(device), LONG_PROJECTION_TILES["gfx950"])
-    share = M / torch.cuda.get_device_properties(device).multi_processor_count
+        tiles = LONG_PROJECTION_TILES.get(arch, LONG_PROJECTION_TILES["gfx950"])
+    share = M / units
     candidates = [tile for most, tile in tiles if share <= most]
     gated = matmul == "gate_up" if gated is None else gated
     residual = matmul == "down" if residual is None else residual
@@ -165,10 +166,11 @@ def takes_rows(device: torch.device, kinds: tuple[str, ...], M: int, K: int) -> 
 def rotate_rows(device: torch.device, M: int) -> int:
     """rotate_quant's rows a wavefront for M rows (reference int8_blocks.py:45-50): the target's ROTATE_ROWS entry for the rows a
     compute unit's share is; a target without one lets the kernel choose."""
-    shares = ROTATE_ROWS.get(gpu_arch(device))
+    arch, units = hip_kernels.gpu(device)
+    shares = ROTATE_ROWS.get(arch)
     if shares is None:
         return UNTIMED_ROTATE_ROWS
-    share = M / torch.cuda.get_device_properties(device).multi_processor_count
+    share = M / units
     return next(rows for most, rows in shares if share <= most)
 
 
