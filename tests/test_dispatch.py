@@ -5,7 +5,7 @@ import math
 import pytest
 import torch
 
-from model import fused_blocks
+from model import fused_blocks, hip_kernels, int8_blocks
 from model.encoding import NUM_SQUARES
 from model.fused_blocks import groups_per_workgroup, move_places, tile_for
 from model.model import ChessTransformer
@@ -16,6 +16,14 @@ def test_tile_for_takes_the_first_row_share_that_fits():
     assert tile_for(tiles, 4 * 256, 256) == 1
     assert tile_for(tiles, 4 * 256 + 1, 256) == 3
     assert tile_for(tiles, 71680, 256) == 11
+
+
+def test_a_projection_table_put_in_the_shipped_ones_place_holds_at_every_depth(monkeypatch):
+    monkeypatch.setattr(hip_kernels, "gpu", lambda device: ("gfx950", 256))
+    chosen = lambda K: int8_blocks.int8_tile(torch.device("cuda"), "projection", 3570, 1152, K, bias=True)
+    assert (chosen(512), chosen(768), chosen(832)) == (11, 6, 11)   # 832: no whole 128-byte lines
+    monkeypatch.setitem(int8_blocks.INT8_TILES["gfx950"], "projection", [(math.inf, 3)])
+    assert (chosen(512), chosen(768)) == (3, 3)
 
 
 @pytest.mark.parametrize("positions", [1, 3, 16, 64, 100, 256, 1024, 4096])
