@@ -93,7 +93,10 @@ _gpus: dict[int, tuple[str, int]] = {}
 
 
 def gpu(device: torch.device) -> tuple[str, int]:
-    """The device's target (gfx950) and its compute units."""
+    """The device's target (gfx950) and its compute units (of anything but a GPU's torch.device, what torch makes of it)."""
+    if not isinstance(device, torch.device) or device.type != "cuda":
+        properties = torch.cuda.get_device_properties(device)
+        return properties.gcnArchName.split(":")[0], properties.multi_processor_count
     index = device.index if device.index is not None else torch.cuda.current_device()
     if index not in _gpus:
         properties = torch.cuda.get_device_properties(index)

@@ -26,6 +26,17 @@ def test_a_projection_table_put_in_the_shipped_ones_place_holds_at_every_depth(m
     assert (chosen(512), chosen(768)) == (3, 3)
 
 
+def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
+    def properties(device):
+        raise ValueError(f"asked about {device}")
+    monkeypatch.setattr(torch.cuda, "get_device_properties", properties)
+    monkeypatch.setattr(hip_kernels, "_gpus", {0: ("gfx950", 256)})
+    assert hip_kernels.gpu(torch.device("cuda", 0)) == ("gfx950", 256)
+    for device in (torch.device("cpu"), "cpu"):
+        with pytest.raises(ValueError, match="asked about cpu"):
+            hip_kernels.gpu(device)
+
+
 @pytest.mark.parametrize("positions", [1, 3, 16, 64, 100, 256, 1024, 4096])
 @pytest.mark.parametrize("kv_heads", [8, 12])
 @pytest.mark.parametrize("tokens", [64, 70, 100])
