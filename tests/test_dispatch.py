@@ -37,6 +37,27 @@ def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
             hip_kernels.gpu(device)
 
 
+@pytest.mark.parametrize("M, K, N, gated, f32, bias, expected", [
+    (256 * 48, 512, 1600, False, False, True, 6), (256 * 48 + 1, 512, 1600, False, False, True, 15),    # the long streams' first row
+    (256 * 49, 512, 1016, False, False, True, 11), (256 * 49, 512, 1024, False, False, True, 15),        # and least columns
+    (256 * 49, 512, 1604, False, False, True, 11), (256 * 49, 512, 1600, False, False, False, 11),       # no whole 8 columns; no bias
+    (256 * 49, 768, 1600, False, False, True, 12), (256 * 101, 768, 768, False, False, True, 13),        # long rows
+    (256 * 9, 704, 512, False, False, True, 3), (256 * 101, 512, 512, True, False, False, 4), (256 * 20, 512, 512, True, False, False, 12),
+    (256 * 9, 512, 512, False, True, False, 1), (256 * 10, 512, 512, False, True, False, 12), (256 * 10, 768, 768, False, True, False, 7),
+    (256 * 10, 32, 512, False, True, False, 7)])                                                          # rows of no whole lines
+def test_linear_picks_its_tile_by_rows_depth_and_epilogue(monkeypatch, M, K, N, gated, f32, bias, expected):
+    chosen = []
+    def launched(x, weight, *arguments):
+        chosen.append(arguments[-1])
+        return x.new_empty(0)
+    monkeypatch.setattr(fused_blocks, "gpu", lambda device: ("gfx950", 256))
+    monkeypatch.setattr(fused_blocks, "launch_linear", launched)
+    width = 2 * N if gated else N
+    x, weight = torch.empty(1, dtype=torch.float16).expand(M, K), torch.empty(K, width, dtype=torch.float16)
+    fused_blocks.linear(x, weight, torch.empty(width, dtype=torch.float16) if bias else None, None, gated, f32)
+    assert chosen == [expected]
+
+
 @pytest.mark.parametrize("positions", [1, 3, 16, 64, 100, 256, 1024, 4096])
 @pytest.mark.parametrize("kv_heads", [8, 12])
 @pytest.mark.parametrize("tokens", [64, 70, 100])
