@@ -40,7 +40,8 @@ RESIDENT_TILE, RESIDENT_DEPTH = 15, 512
 # column groups and output bytes it takes
 RESIDENT_WIDE_SHARE, RESIDENT_WIDE_COLUMNS = 48, range(1024, 4097)
 # gated: at 512 to 2 x 2,048 (graphs of launches, us) 4,480 rows take 27.0 on tile 12 and 29.6 on tile 6, 35,840 rows 172.8 on
-# the eight-wavefront 256 x 128 tile 4 and 175.6 on tile 11, 71,680 rows 333 and 336; 768 to 2 x 992 at 49,000 rows 167 and 181
+# the eight-wavefront 256 x 128 tile 4 and 175.6 on tile 11, 71,680 rows 333 and 336; 768 to 2 x 992 at 49,000 rows 167 and 181.
+# Rows of whole lines only (tile 12 stages 128 bytes of a row); others keep LINEAR_TILES
 LINEAR_GATED_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (100, 11), (math.inf, 4)]}
 # f32 out (accumulate_fp32, the policy head's `a`), graphs of launches on an MI355X, us: rows shorter than LONG_ROW_BYTES and of
 # whole lines take 128 x 64 with 128-byte stages (512 to 512: 9.2 against 10.5 on tile 7 at 4,480 rows, 25.0 against 32.1 at
@@ -75,11 +76,12 @@ def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: b
 
 def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False) -> int:
     arch, units = gpu(device)
+    whole_lines = row_bytes % 128 == 0
     if accumulate_fp32:
-        table = LINEAR_F32_TILES if row_bytes % 128 == 0 and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
-    elif gated:
+        table = LINEAR_F32_TILES if whole_lines and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
+    elif gated and whole_lines:
         table = LINEAR_GATED_TILES
-    elif row_bytes >= LONG_ROW_BYTES and row_bytes % 128 == 0:
+    elif row_bytes >= LONG_ROW_BYTES and whole_lines and not gated:
         table = LINEAR_LONG_ROW_TILES
     else:
         table = LINEAR_TILES

@@ -44,7 +44,8 @@ def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
     (256 * 49, 768, 1600, False, False, True, 12), (256 * 101, 768, 768, False, False, True, 13),        # long rows
     (256 * 9, 704, 512, False, False, True, 3), (256 * 101, 512, 512, True, False, False, 4), (256 * 20, 512, 512, True, False, False, 12),
     (256 * 9, 512, 512, False, True, False, 1), (256 * 10, 512, 512, False, True, False, 12), (256 * 10, 768, 768, False, True, False, 7),
-    (256 * 10, 32, 512, False, True, False, 7)])                                                          # rows of no whole lines
+    (256 * 10, 32, 512, False, True, False, 7),                                                          # rows of no whole lines
+    (256 * 10, 96, 512, True, False, False, 6), (256 * 20, 544, 512, True, False, False, 6), (256 * 101, 96, 512, True, False, False, 0)])
 def test_linear_picks_its_tile_by_rows_depth_and_epilogue(monkeypatch, M, K, N, gated, f32, bias, expected):
     chosen = []
     def launched(x, weight, *arguments):
@@ -56,6 +57,17 @@ def test_linear_picks_its_tile_by_rows_depth_and_epilogue(monkeypatch, M, K, N, 
     x, weight = torch.empty(1, dtype=torch.float16).expand(M, K), torch.empty(K, width, dtype=torch.float16)
     fused_blocks.linear(x, weight, torch.empty(width, dtype=torch.float16) if bias else None, None, gated, f32)
     assert chosen == [expected]
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("gated", [False, True])
+def test_linear_picks_no_tile_that_refuses_its_rows(monkeypatch, f32, gated):
+    """Tiles 5, 12 and 13 stage 128 bytes of a row at a time and refuse rows of no whole 128 bytes; linear takes any multiple of 32
+    inputs (64 bytes), at every share of rows."""
+    monkeypatch.setattr(fused_blocks, "gpu", lambda device: ("gfx950", 256))
+    for K in range(32, 2112, 32):
+        for M in (1, 256 * 4, 256 * 5, 256 * 9, 256 * 10, 256 * 20, 256 * 21, 256 * 48, 256 * 49, 256 * 75, 256 * 100, 256 * 101):
+            assert K % 64 == 0 or fused_blocks.linear_tile(torch.device("cuda"), M, f32, 2 * K, gated) not in (5, 12, 13), (M, K)
 
 
 @pytest.mark.parametrize("positions", [1, 3, 16, 64, 100, 256, 1024, 4096])

@@ -834,6 +834,17 @@ def test_linear_gated_mixed_and_fp32(device):
     assert np.allclose(cpu(wide), cpu(x).astype(np.float64) @ cpu(gate_up).astype(np.float64), atol=1e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize("M, K, N", [(2560, 96, 72), (5120, 160, 64), (26112, 96, 72)])
+def test_gated_linear_takes_rows_of_no_whole_lines(device, M, K, N):
+    """Rows of a multiple of 64 bytes but not of 128, at the shares of rows where longer ones take tiles that stage 128 bytes of a
+    row; the tolerances of the gated launch above."""
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device=device).half()
+    gate_up = (torch.randn(K, 2 * N, device=device) / math.sqrt(K)).half()
+    expected = oracle.linear(cpu(x), cpu(gate_up), gated=True).astype(np.float64)
+    assert np.allclose(cpu(linear(x, gate_up, gated=True)).astype(np.float64), expected, atol=2e-3, rtol=4e-3)
+
+
 def test_the_kernels_run_in_graphs_on_two_streams(device):
     """The reference's isolation check (tests/test_int8.py:161-184, tests/test_attention_cuda.py:110-130): two graphs replayed
     together on two streams give the eager bits."""
