@@ -76,7 +76,7 @@ def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: b
 
 def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False) -> int:
     arch, units = gpu(device)
-    whole_lines = row_bytes % 128 == 0
+    whole_lines = row_bytes > 0 and row_bytes % 128 == 0   # (0: the rows' length is not known)
     if accumulate_fp32:
         table = LINEAR_F32_TILES if whole_lines and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
     elif gated and whole_lines:

@@ -70,6 +70,15 @@ def test_linear_picks_no_tile_that_refuses_its_rows(monkeypatch, f32, gated):
             assert K % 64 == 0 or fused_blocks.linear_tile(torch.device("cuda"), M, f32, 2 * K, gated) not in (5, 12, 13), (M, K)
 
 
+def test_linear_tiles_for_rows_of_unknown_length_take_any_row(monkeypatch):
+    """linear_tile asked without the rows' bytes names a tile that takes rows of any length."""
+    monkeypatch.setattr(fused_blocks, "gpu", lambda device: ("gfx950", 256))
+    for M in (1, 256 * 5, 256 * 10, 256 * 21, 256 * 49, 256 * 101):
+        for f32, gated in ((False, False), (False, True), (True, False), (True, True)):
+            assert fused_blocks.linear_tile(torch.device("cuda"), M, f32, gated=gated) not in (5, 12, 13), (M, f32, gated)
+    assert fused_blocks.linear_tile(torch.device("cuda"), 256 * 10, True) == 7
+
+
 @pytest.mark.parametrize("positions", [1, 3, 16, 64, 100, 256, 1024, 4096])
 @pytest.mark.parametrize("kv_heads", [8, 12])
 @pytest.mark.parametrize("tokens", [64, 70, 100])
