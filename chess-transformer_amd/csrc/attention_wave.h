@@ -149,7 +149,9 @@ void template_attention_wave_kernel(
         return __builtin_bit_cast(v8h, uint4{normed[0], normed[1], normed[2], normed[3]});
     };
     // A position's rows as a buffer: a load takes the lane's part of its address from a register and the rest from a scalar
-    // one. Rows past T lie past the buffer and read as zeros (their scores are masked, their outputs not stored).
+    // one. Of the tile past the squares, whose rows may pass T, the whole row is in the lane's part, held to row T - 1 (such a
+    // row's scores are masked, its outputs not stored): every load is inside the rows, whatever of an address a buffer's bounds
+    // check counts.
     const uint32_t row_bytes = (uint32_t)width * 2;
     auto rows_of = [&](int pair) {
         return buffer_resource(projected + (size_t)(pair / kv_heads) * T * width, (uint32_t)T * row_bytes);
@@ -157,6 +159,7 @@ void template_attention_wave_kernel(
     uint32_t lane_row[KS];   // the lane's chunks of row col
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) lane_row[ks] = (uint32_t)col * row_bytes + (uint32_t)chunk[ks] * 2;
+    const uint32_t to_tail = (uint32_t)(min(64 + col, T - 1) - col) * row_bytes;   // from there to row 64 + col's
     uint4 raw_keys[TILES][KS];
     auto load_keys = [&](int pair) {
         const BufferResource rows = rows_of(pair);
@@ -164,18 +167,20 @@ void template_attention_wave_kernel(
 #pragma unroll
         for (int kt = 0; kt < TILES; kt++)
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) raw_keys[kt][ks] = buffer_load16(rows, lane_row[ks], at + kt * 16 * row_bytes);
+            for (int ks = 0; ks < KS; ks++)
+                raw_keys[kt][ks] = kt < 4 ? buffer_load16(rows, lane_row[ks], at + kt * 16 * row_bytes) : buffer_load16(rows, lane_row[ks] + to_tail, at);
     };
     // a slab's query rows and template coefficients of head hi of a pair's
     uint4 raw_query[KS], raw_mix;
     auto load_query = [&](int pair, int hi, int slab) {
         const BufferResource rows = rows_of(pair);
         const int head = pair % kv_heads * per_kv + hi;
-        const uint32_t at = (uint32_t)slab * 16 * row_bytes;
+        const bool past = TILES > 4 && slab == 4;
+        const uint32_t at = past ? 0 : (uint32_t)slab * 16 * row_bytes, shift = past ? to_tail : 0;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) raw_query[ks] = buffer_load16(rows, lane_row[ks], at + (uint32_t)(head * dq) * 2);
+        for (int ks = 0; ks < KS; ks++) raw_query[ks] = buffer_load16(rows, lane_row[ks] + shift, at + (uint32_t)(head * dq) * 2);
         if (templates_count == MAX_TEMPLATES) {
-            raw_mix = buffer_load16(rows, (uint32_t)col * row_bytes, at + (uint32_t)(c_offset + head * MAX_TEMPLATES) * 2);
+            raw_mix = buffer_load16(rows, (uint32_t)col * row_bytes + shift, at + (uint32_t)(c_offset + head * MAX_TEMPLATES) * 2);
         } else {   // fewer than 8 coefficients start at any 2-byte place (past the squares a square's are read, and not used)
             const half_t* from = projected + ((size_t)(pair / kv_heads) * T + min(slab * 16 + col, 63)) * width + c_offset + head * templates_count;
             uint16_t c[MAX_TEMPLATES];
@@ -195,9 +200,10 @@ void template_attention_wave_kernel(
             // streamed (WHOLE): the values are read once, and past the caches they leave the output rows there for the combine
             // GEMM (67.1 against 70.4 us at batch 1024; the keys' and queries' rows, whose lines other heads read too, streamed
             // as well: 77.3)
-            const uint32_t lane_at = (uint32_t)((i + 1) * DMA_ROWS <= 64 ? lane_slot : min(row, T - 1) - i * DMA_ROWS) * row_bytes + c * 16;
-            if constexpr (MODE == WHOLE) buffer_dma16_streamed(rows, (LDS_SPACE void*)(values + i * 1024), lane_at, at + i * DMA_ROWS * row_bytes);
-            else buffer_dma16(rows, (LDS_SPACE void*)(values + i * 1024), lane_at, at + i * DMA_ROWS * row_bytes);
+            const bool squares = (i + 1) * DMA_ROWS <= 64;
+            const uint32_t lane_at = (uint32_t)(squares ? lane_slot : min(row, T - 1)) * row_bytes + c * 16, row_at = squares ? i * DMA_ROWS * row_bytes : 0;
+            if constexpr (MODE == WHOLE) buffer_dma16_streamed(rows, (LDS_SPACE void*)(values + i * 1024), lane_at, at + row_at);
+            else buffer_dma16(rows, (LDS_SPACE void*)(values + i * 1024), lane_at, at + row_at);
         }
     };
     // the templates of the wavefront's own slab, in the steps' order (FOURS and SLABS)
@@ -454,7 +460,10 @@ void template_attention_wave_kernel(
                 words[dt] = uint2{narrow16x2<BF16>(o[dt][0] * inverse_total, o[dt][1] * inverse_total),
                                   narrow16x2<BF16>(o[dt][2] * inverse_total, o[dt][3] * inverse_total)};
             const BufferResource outs = buffer_resource(out + (size_t)(pair / kv_heads) * T * (heads * DV), (uint32_t)(T * heads * DV) * 2);
-            const uint32_t at = (uint32_t)((slab * 16 * heads + head) * DV) * 2, lane_at = (uint32_t)(col * heads * DV) * 2;
+            // (past the squares as the loads: the whole row in the lane's part, and for rows past T a part past any buffer,
+            // which stores nothing)
+            const uint32_t out_bytes = (uint32_t)(heads * DV) * 2, at = (SQUARES ? (uint32_t)slab * 16 * out_bytes : 0) + (uint32_t)(head * DV) * 2;
+            const uint32_t lane_at = SQUARES ? col * out_bytes : 64 + col < T ? (64 + col) * out_bytes : 0x80000000u;
             if constexpr (DT == 1) {
                 buffer_store8(outs, words[0], lane_at + quad * 8, at);
             } else {

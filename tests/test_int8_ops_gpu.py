@@ -13,6 +13,7 @@ import torch.nn.functional as F
 
 from oracle import int8_ops as oracle
 from model import fused_blocks, int8_blocks
+from model.hip_kernels import check, library_for, pointer, stream_of
 from model.int8_blocks import (HADAMARD_BLOCK, INT8_TILES, hadamard, int8_linear, int8_matmul_i32, launch_int8_linear, mix_norm_quant, norm_quant,
                                rotate_quant)
 from model.fused_blocks import launch_linear, launch_template_attention, linear, mix_rms_norm, rms_norm, template_attention
@@ -747,6 +748,32 @@ def test_both_sharings_of_the_pairs_give_the_same_bits(device, heads, kv_heads, 
         kept = [k for k, position in enumerate(rows) if position in set(clean)]
         out = template_attention(spoilt[rows].contiguous(), *arguments[1:])
         assert torch.equal(out[kept], whole[[rows[k] for k in kept]])
+
+
+@pytest.mark.parametrize("tokens", [64, 65, 70, 72, 73, 80])
+@pytest.mark.parametrize("heads, kv_heads, dq, dv, count", [(4, 4, 64, 64, 8), (6, 3, 24, 32, 8), (2, 2, 40, 16, 4)])
+def test_attention_reads_and_writes_nothing_past_its_rows(device, tokens, heads, kv_heads, dq, dv, count):
+    """Up to 80 tokens, widths up to 64: the last tiles of 16 rows reach past a position's tokens. With NaNs round the input rows
+    (and in LDS, left by a launch before) and a sentinel round the outputs, at the C entry: the fp32 formula's answer, the operator's
+    bits, and every sentinel as it was, whether the wavefronts take whole pairs (the large launch) or share one."""
+    units = torch.cuda.get_device_properties(device).multi_processor_count
+    library, guard, sentinel = library_for(device), 128 * 1024, 12345.0
+    for positions in (3, 6 * units // kv_heads + 2):
+        arguments = attention_operands(device, positions, heads, kv_heads, dq, dv, seed=tokens + dq, tokens=tokens, templates_count=count)
+        projected, templates, q_gain, k_gain = arguments[:4]
+        rows = torch.full((guard + projected.numel() + guard,), float("nan"), device=device, dtype=torch.float16)
+        rows[guard:-guard] = projected.flatten()
+        outputs = positions * tokens * heads * dv
+        out = torch.full((guard + outputs + guard,), sentinel, device=device, dtype=torch.float16)
+        keyed = fused_blocks.keyed_templates(templates, count)
+        template_attention(torch.full_like(projected, float("nan")), *arguments[1:])
+        at = lambda buffer: pointer(buffer[guard:])
+        check(library.chess_template_attention(at(rows), pointer(keyed), pointer(q_gain), pointer(k_gain), at(out), positions, tokens, heads, kv_heads,
+                                               dq, dv, count, 1, EPS, 1 / math.sqrt(dq), stream_of(device)), "template_attention")
+        found = out[guard:-guard].view(positions, tokens, heads * dv)
+        assert torch.allclose(found.float(), reference_attention(arguments), atol=1e-2)
+        assert torch.equal(found, template_attention(*arguments))
+        assert (out[:guard] == sentinel).all() and (out[-guard:] == sentinel).all()
 
 
 def bf16_operands(arguments):
