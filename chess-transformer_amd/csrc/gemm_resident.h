@@ -27,6 +27,7 @@
 #include "gemm.h"
 #include "lds_dma.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace resident {
@@ -401,9 +402,28 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));   // the tail's repeated DMA lands before the LDS is reused
 }
 
-// The launch: a workgroup a compute unit, each XCD's workgroups taking streams of row blocks for every column group. A last
-// group with columns for only some wavefronts gets fewer workgroups and longer streams: its turns cost about
-// (WAVES + working wavefronts) / (2 WAVES) of a full group's.
+// How an XCD's workgroups are shared out: `slices` streams of row blocks for every column group but the last, which has
+// `last_slices`. A last group with columns for only some wavefronts (they idle, but not beside a residual) gets fewer
+// workgroups and longer streams: its turns cost about (WAVES + working wavefronts) / (2 WAVES) of a full group's. Of all such
+// shares the one whose longest stream is the shortest: rounding the full groups' share up instead can leave the last group
+// almost none (256 to 2 x 1,408: six and two of 32, where five and seven take 0.200 of the rows' time and not 0.375). Graphs of
+// launches on an MI355X, us, rounded up and so: 70,000 rows of 256 to 2 x 1,408 120.7 and 83.0, of 512 to 2 x 1,408 145.0 and
+// 106.8; 35,000 of 1,024 to 1,600 80.2 and 64.4; 69,930 of 768 to 1,152 73.4 and 69.3; 512 to 1,600 (nine and five) is shared alike.
+struct Plan { int groups, slices, last_slices; };
+template <typename S> Plan plan(int N, int per_xcd) {
+    Plan p{(N + S::GROUP - 1) / S::GROUP, 0, 0};
+    p.slices = p.last_slices = per_xcd / p.groups;
+    const int working = (N - (p.groups - 1) * S::GROUP + S::COLUMNS - 1) / S::COLUMNS;   // the last group's working wavefronts
+    if (p.groups == 1 || working == WAVES || S::RESIDUAL) return p;
+    const double cost = (WAVES + working) / (2.0 * WAVES);
+    auto longest = [&](int slices) { return std::max(1.0 / slices, cost / (per_xcd - (p.groups - 1) * slices)); };
+    for (int slices = p.slices + 1; slices <= (per_xcd - 1) / (p.groups - 1); slices++)
+        if (longest(slices) < longest(p.slices)) p.slices = slices;
+    p.last_slices = per_xcd - (p.groups - 1) * p.slices;
+    return p;
+}
+
+// The launch: a workgroup a compute unit, each XCD's workgroups taking streams of row blocks for every column group.
 template <typename In, int NB, typename OutT, int EPI, int DEPTH_ = DEPTH>
 int launch(const void* x, const void* w, void* out, const Epilogue& e, int M, int N, hipStream_t stream) {
     typedef Shape<In, NB, EPI, DEPTH_> S;
@@ -417,15 +437,9 @@ int launch(const void* x, const void* w, void* out, const Epilogue& e, int M, in
     const int per_xcd = workgroups / XCDS, groups = (N + S::GROUP - 1) / S::GROUP;
     if (groups > per_xcd)
         return chess_fail(CHESS_UNSUPPORTED, "tile 15 takes at most %d column groups of %d on this device, not %d", per_xcd, S::GROUP, groups);
-    const int working = (N - (groups - 1) * S::GROUP + S::COLUMNS - 1) / S::COLUMNS;   // the last group's working wavefronts
-    int slices = per_xcd / groups, last_slices = slices;
-    if (groups > 1 && working < WAVES && !S::RESIDUAL) {
-        const double cost = (WAVES + working) / (2.0 * WAVES);
-        slices = min((int)(per_xcd / (groups - 1 + cost) + 0.5), (per_xcd - 1) / (groups - 1));
-        last_slices = per_xcd - (groups - 1) * slices;
-    }
-    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * WAVES), S::LDS_BYTES, stream, (const In*)x, (const In*)w, (OutT*)out, e, M, N, groups,
-                       slices, last_slices);
+    const Plan p = plan<S>(N, per_xcd);
+    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * WAVES), S::LDS_BYTES, stream, (const In*)x, (const In*)w, (OutT*)out, e, M, N, p.groups,
+                       p.slices, p.last_slices);
     return launch_status();
 }
 

@@ -466,11 +466,13 @@ def test_the_register_tile_at_the_batch_1024_rows(device):
 
 @pytest.mark.parametrize("matmul, depth, width", [("projection", 256, 520), ("projection", 512, 520), ("projection", 768, 1032),
                                                   ("projection", 1024, 264), ("gate_up", 256, 264), ("gate_up", 768, 136),
-                                                  ("down", 1024, 264), ("mixing down", 1024, 264)])
+                                                  ("down", 1024, 264), ("mixing down", 1024, 264), ("projection", 768, 1152),
+                                                  ("projection", 1024, 1600), ("gate_up", 256, 1408)])
 @pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16])
 def test_large_launches_of_tile_0_give_the_whole_k_tiles_bits(device, matmul, depth, width, out_dtype):
     """Tile 0 holds the weights in registers where a workgroup's stream of row blocks is long: 41,007 rows (past each
-    epilogue's line; a ragged last block and a column group part past N) against tile 1, at every depth it has."""
+    epilogue's line; a ragged last block and a column group part past N) against tile 1, at every depth it has; five to seven
+    column groups, the last part past N and with more streams than each of the others."""
     x, x_scale, weight, weight_scale, bias, residual, gated, mix = int8_operands(matmul, 41007, device, width=width, depth=depth)
     found = launch_int8_linear(x, x_scale, weight, weight_scale, bias, residual, gated, *mix, 0, out_dtype)
     assert same_bits(found, launch_int8_linear(x, x_scale, weight, weight_scale, bias, residual, gated, *mix, 1, out_dtype))
