@@ -409,17 +409,21 @@ __global__ __launch_bounds__(64 * WAVES, 1) void resident_kernel(
 // almost none (256 to 2 x 1,408: six and two of 32, where five and seven take 0.200 of the rows' time and not 0.375). Graphs of
 // launches on an MI355X, us, rounded up and so: 70,000 rows of 256 to 2 x 1,408 120.7 and 83.0, of 512 to 2 x 1,408 145.0 and
 // 106.8; 35,000 of 1,024 to 1,600 80.2 and 64.4; 69,930 of 768 to 1,152 73.4 and 69.3; 512 to 1,600 (nine and five) is shared alike.
-struct Plan { int groups, slices, last_slices; };
+// `busy` is the part of the XCD's workgroups' time that the groups' work takes.
+struct Plan { int groups, slices, last_slices; double busy; };
 template <typename S> Plan plan(int N, int per_xcd) {
-    Plan p{(N + S::GROUP - 1) / S::GROUP, 0, 0};
+    Plan p{(N + S::GROUP - 1) / S::GROUP};
     p.slices = p.last_slices = per_xcd / p.groups;
     const int working = (N - (p.groups - 1) * S::GROUP + S::COLUMNS - 1) / S::COLUMNS;   // the last group's working wavefronts
-    if (p.groups == 1 || working == WAVES || S::RESIDUAL) return p;
-    const double cost = (WAVES + working) / (2.0 * WAVES);
-    auto longest = [&](int slices) { return std::max(1.0 / slices, cost / (per_xcd - (p.groups - 1) * slices)); };
-    for (int slices = p.slices + 1; slices <= (per_xcd - 1) / (p.groups - 1); slices++)
-        if (longest(slices) < longest(p.slices)) p.slices = slices;
-    p.last_slices = per_xcd - (p.groups - 1) * p.slices;
+    const double cost = (WAVES + working) / (2.0 * WAVES), last_cost = S::RESIDUAL ? 1.0 : cost;
+    auto longest = [&](int slices, int last_slices) { return std::max(p.groups > 1 ? 1.0 / slices : 0.0, last_cost / last_slices); };
+    if (p.groups > 1 && last_cost < 1.0) {
+        auto last_of = [&](int slices) { return per_xcd - (p.groups - 1) * slices; };
+        for (int slices = p.slices + 1; slices <= (per_xcd - 1) / (p.groups - 1); slices++)
+            if (longest(slices, last_of(slices)) < longest(p.slices, last_of(p.slices))) p.slices = slices;
+        p.last_slices = last_of(p.slices);
+    }
+    p.busy = (p.groups - 1 + cost) / per_xcd / longest(p.slices, p.last_slices);
     return p;
 }
 
@@ -506,7 +510,15 @@ template <typename In, int NB, typename OutT, typename F> bool taken(int flags, 
 // weight row that writes more than the last-level cache's 256 MB is bound by its writes, and whole lines from LDS go faster
 // than these 16-byte stores (512 to 2,048 at 65,536 rows, 268 MB: 121 us and 109 on tile 4; 512 to 1,600 at 71,680, 229 MB: 89
 // and 105); gated, 293 MB still take 163 and 240.
-constexpr int STREAM_BLOCKS = 10, DEEP_STREAM_BLOCKS = 6, F16_STREAM_BLOCKS = 8;
+// Below LARGE_ROWS, where the other tile is 11 and not the slower 4, a plan whose workgroups are too often out of work does not
+// pay: 768 to 2 x 2,176 (17 groups for 32 workgroups, busy 0.53) at 12,000 rows 68.5 and 59.9, 256 to 2 x 4,352 65.9 and 49.1 (at
+// 35,000 177 and 174, at 70,000 345 and 333; 512 to 2 x 4,352 208 and 241), 512 to 2 x 2,816 (11 groups, 0.69) 49.8 and 52.5; with the
+// shorter MFMA chains of depth 256 the line lies higher, 256 to 2 x 2,816 39.6 and 34.1. Two working wavefronts of a sole group's
+// eight do not either: 256 to 72 at 110,000 rows 18.4 and 14.1, 512 to 72 19.8 and 19.0 (three, 768 to 72: 20.9 and 23.4). Beside a
+// residual a part-filled group costs a full one, which near the line is no loss yet: 1,024 to 264 and 384 at 25,000 rows 22.9
+// and 24.1, where tile 13 takes 23.9 and 24.3; with the mix 27.0 and 29.2, and 26.9 and 27.9.
+constexpr int STREAM_BLOCKS = 10, DEEP_STREAM_BLOCKS = 6, F16_STREAM_BLOCKS = 8, LARGE_ROWS = 32768;
+constexpr double LEAST_BUSY = 0.6, LEAST_BUSY_256 = 0.7;
 constexpr uint64_t MOST_WRITTEN = 256ull << 20;
 
 template <typename In, int NB, typename OutT> bool takes(int flags, int M, int N, int K) {
@@ -516,9 +528,11 @@ template <typename In, int NB, typename OutT> bool takes(int flags, int M, int N
     bool worth = false;
     const bool known = taken<In, NB, OutT>(flags, K, [&](auto depth, auto epilogue) {
         typedef Shape<In, NB, decltype(epilogue)::value, decltype(depth)::value> S;
-        const int groups = (N + S::GROUP - 1) / S::GROUP;
-        const int least = !S::INT8 ? F16_STREAM_BLOCKS : S::RESIDUAL ? DEEP_STREAM_BLOCKS : STREAM_BLOCKS;
-        worth = groups <= units / XCDS && (long)(M / ROWS) * groups >= (long)least * units;
+        const int per_xcd = units / XCDS, least = !S::INT8 ? F16_STREAM_BLOCKS : S::RESIDUAL ? DEEP_STREAM_BLOCKS : STREAM_BLOCKS;
+        if ((N + S::GROUP - 1) / S::GROUP > per_xcd || N <= 2 * S::COLUMNS) return;
+        const Plan p = plan<S>(N, per_xcd);
+        worth = (M >= LARGE_ROWS || p.busy >= (S::ROW_BYTES == 256 ? LEAST_BUSY_256 : LEAST_BUSY))
+             && (long)(M / ROWS) * p.groups >= (long)least * units;
     });
     return known && worth;
 }
