@@ -507,9 +507,13 @@ template <typename In, int NB, typename OutT, typename F> bool taken(int flags, 
 // 17,920 (4) 14.9 and 11.7, 69,930 (17) 31.6 and 35.4; 1,024 to 768 with the residual and the mix, 17,920 (7) 29.4 and 32.2,
 // 35,000 (13) 46.8 and 54.4; 1,024 to 256 so, 35,000 (4) 25.7 and 25.0, 69,930 (9) 36.5 and 41.1; fp16, 256 to 256 with bias
 // and residual, 69,930 (9) 22.4 and 24.5. (Left out, as no faster: the residual at depths 512 and 768.) A launch of one output a
-// weight row that writes more than the last-level cache's 256 MB is bound by its writes, and whole lines from LDS go faster
-// than these 16-byte stores (512 to 2,048 at 65,536 rows, 268 MB: 121 us and 109 on tile 4; 512 to 1,600 at 71,680, 229 MB: 89
-// and 105); gated, 293 MB still take 163 and 240.
+// weight row that writes more than the last-level cache holds is bound by its writes, and whole lines from LDS go faster than
+// these 16-byte stores (512 to 2,048 at 65,536 rows, 268 MB: 121 us and 109 on tile 4); gated, 293 MB still take 163 and 240. For
+// output rows of whole KB, whose 32 rows a store falls on few of L2's channels, from short inputs and without a residual to
+// read that is so from 230 MiB on (this kernel and tile 4: 512 to 1,024, 210 MiB 90 and 92, 230 MiB 116 and 100; 512 to 1,536, 220
+// MiB 95 and 95, 240 MiB 115 and 100; 512 to 2,048, 230 MiB 99 and 100, 255 MiB 120 and 110; 256 to 2,048, 240 MiB 73 and 76, 250
+// MiB 84 and 77), for others not up to 256 MiB (512 to 1,600, 230 MiB 80 and 103, 255 MiB 106 and 116; 768 to 1,152, 255 MiB 139
+// and 150; 1,024 to 1,024 with the residual 163 and 239; fp16, 512 to 512 144 and 195).
 // Below LARGE_ROWS, where the other tile is 11 and not the slower 4, a plan whose workgroups are too often out of work does not
 // pay: 768 to 2 x 2,176 (17 groups for 32 workgroups, busy 0.53) at 12,000 rows 68.5 and 59.9, 256 to 2 x 4,352 65.9 and 49.1 (at
 // 35,000 177 and 174, at 70,000 345 and 333; 512 to 2 x 4,352 208 and 241), 512 to 2 x 2,816 (11 groups, 0.69) 49.8 and 52.5; with the
@@ -519,10 +523,13 @@ template <typename In, int NB, typename OutT, typename F> bool taken(int flags, 
 // and 24.1, where tile 13 takes 23.9 and 24.3; with the mix 27.0 and 29.2, and 26.9 and 27.9.
 constexpr int STREAM_BLOCKS = 10, DEEP_STREAM_BLOCKS = 6, F16_STREAM_BLOCKS = 8, LARGE_ROWS = 32768;
 constexpr double LEAST_BUSY = 0.6, LEAST_BUSY_256 = 0.7;
-constexpr uint64_t MOST_WRITTEN = 256ull << 20;
+constexpr uint64_t MOST_WRITTEN = 256ull << 20, MOST_WRITTEN_WHOLE_KB = 230ull << 20;
 
 template <typename In, int NB, typename OutT> bool takes(int flags, int M, int N, int K) {
-    if (N % 8 != 0 || (uint64_t)M * N * sizeof(OutT) >= (NB == 1 ? MOST_WRITTEN : 1ull << 31)) return false;
+    const uint64_t row_bytes = (uint64_t)N * sizeof(OutT);
+    const bool short_inputs = (size_t)K * sizeof(In) <= 512 && !(flags & EPI_RESIDUAL);
+    const uint64_t most = NB == 2 ? 1ull << 31 : short_inputs && row_bytes % 1024 == 0 ? MOST_WRITTEN_WHOLE_KB : MOST_WRITTEN;
+    if (N % 8 != 0 || M * row_bytes >= most) return false;
     int device = 0, units = 0;
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return false;
     bool worth = false;
