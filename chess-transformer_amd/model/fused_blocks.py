@@ -39,10 +39,15 @@ RESIDENT_TILE, RESIDENT_DEPTH = 15, 512
 # blocks (512 to 1,600 columns at 17,920 rows, graphs of launches: 37.4 against 43.0 us on tile 11); up to 4,096, inside the
 # column groups and output bytes it takes
 RESIDENT_WIDE_SHARE, RESIDENT_WIDE_COLUMNS = 48, range(1024, 4097)
-# gated: at 512 to 2 x 2,048 (graphs of launches, us) 4,480 rows take 27.0 on tile 12 and 29.6 on tile 6, 35,840 rows 172.8 on
-# the eight-wavefront 256 x 128 tile 4 and 175.6 on tile 11, 71,680 rows 333 and 336; 768 to 2 x 992 at 49,000 rows 167 and 181.
-# Rows of whole lines only (tile 12 stages 128 bytes of a row); others keep LINEAR_TILES
-LINEAR_GATED_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (100, 11), (math.inf, 4)]}
+# gated, rows of whole lines (tile 12 stages 128 bytes of a row) from 1 KB on; others keep LINEAR_TILES. Graphs of launches, us:
+# 512 to 2 x 2,048 4,480 rows 27.5 on tile 12 and 29.3 on tile 6, 1,024 to 2 x 2,816 63.3 and 69.7, but 256 to 2 x 1,024 12.1 and
+# 11.7. Past 100 rows a compute unit the eight-wavefront 256 x 128 tile 4 pays for rows of 1,408 bytes or more (tile 4 and 11; 32,000
+# and 71,680 rows): 704 to 2 x 2,048 196 and 204, 443 and 444; 768 to 2 x 992 107 and 115, 236 and 249; 1,024 to 2 x 2,816 361 and 385,
+# 797 and 842; but 512 to 2 x 2,048 153 and 151, 345 and 328; 512 to 2 x 512 at 35,840 rows 56.3 and 48.8; 256 to 2 x 1,024 49.2 and
+# 44.6, 104 and 95; 640 to 2 x 1,280 either way
+LINEAR_GATED_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (math.inf, 11)]}
+LINEAR_GATED_LONG_ROW_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (100, 11), (math.inf, 4)]}
+GATED_ROW_BYTES, GATED_LONG_ROW_BYTES = 1024, 1408
 # f32 out (accumulate_fp32, the policy head's `a`), graphs of launches on an MI355X, us: rows shorter than LONG_ROW_BYTES and of
 # whole lines take 128 x 64 with 128-byte stages (512 to 512: 9.2 against 10.5 on tile 7 at 4,480 rows, 25.0 against 32.1 at
 # 17,920, 78.6 against 83.7 at 71,680) and 64 x 64 up to 9 rows a compute unit (1,120 rows 5.6 against 9.4); longer ones the
@@ -79,8 +84,8 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
     whole_lines = row_bytes > 0 and row_bytes % 128 == 0   # (0: the rows' length is not known)
     if accumulate_fp32:
         table = LINEAR_F32_TILES if whole_lines and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
-    elif gated and whole_lines:
-        table = LINEAR_GATED_TILES
+    elif gated and whole_lines and row_bytes >= GATED_ROW_BYTES:
+        table = LINEAR_GATED_TILES if row_bytes < GATED_LONG_ROW_BYTES else LINEAR_GATED_LONG_ROW_TILES
     elif row_bytes >= LONG_ROW_BYTES and whole_lines and not gated:
         table = LINEAR_LONG_ROW_TILES
     else:
