@@ -48,12 +48,14 @@ RESIDENT_WIDE_SHARE, RESIDENT_WIDE_COLUMNS = 48, range(1024, 4097)
 LINEAR_GATED_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (math.inf, 11)]}
 LINEAR_GATED_LONG_ROW_TILES = {"gfx950": [(5, 1), (9, 3), (20, 12), (48, 6), (100, 11), (math.inf, 4)]}
 GATED_ROW_BYTES, GATED_LONG_ROW_BYTES = 1024, 1408
-# f32 out (accumulate_fp32, the policy head's `a`), graphs of launches on an MI355X, us: rows shorter than LONG_ROW_BYTES and of
-# whole lines take 128 x 64 with 128-byte stages (512 to 512: 9.2 against 10.5 on tile 7 at 4,480 rows, 25.0 against 32.1 at
-# 17,920, 78.6 against 83.7 at 71,680) and 64 x 64 up to 9 rows a compute unit (1,120 rows 5.6 against 9.4); longer ones the
-# 128 x 128 with a 3-stage ring (768 to 768 at 21,000 rows: 53.6 against 57.1)
+# f32 out (accumulate_fp32, the policy head's `a`), graphs of launches on an MI355X, us: rows of whole lines up to 2 KB take
+# 128 x 64 with 128-byte stages (512 to 512: 9.3 against 10.8 on tile 7 at 4,480 rows, 24.5 against 33.7 at 17,920, 78.8 against
+# 84.7 at 71,680; 768 to 768 11.5 against 13.5 at 3,570, 50.4 against 52.9 at 21,000; 1,024 to 1,024 71.8 against 81.3 there) and
+# 64 x 64 up to 9 rows a compute unit (1,120 rows 5.7 against 9.5, 7.1 against 11.8 and 8.9 against 14.3); others the 128 x 128
+# with a 3-stage ring
 LINEAR_F32_TILES = {"gfx950": [(9, 1), (math.inf, 12)]}
-LINEAR_F32_LONG_ROW_TILES = {"gfx950": [(4, 1), (math.inf, 7)]}
+LINEAR_F32_OTHER_TILES = {"gfx950": [(4, 1), (math.inf, 7)]}
+F32_ROW_BYTES = 2048
 # rows of 1.5 KB or more (the fp16 block's down, combine of a width of 768 or more), not gated: 128 x 128 with 128-byte stages,
 # whole L2 lines a step (2,048 inputs: 190 against 226 us at 71,680 rows, 94 against 101 with tile 12 at 35,840; 768 inputs to
 # 768: 79.2 against 91.9 with tile 11 at 49,000); 128 x 64 with 128-byte stages up to 100 rows a compute unit (2,048 inputs at
@@ -83,7 +85,7 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
     arch, units = gpu(device)
     whole_lines = row_bytes > 0 and row_bytes % 128 == 0   # (0: the rows' length is not known)
     if accumulate_fp32:
-        table = LINEAR_F32_TILES if whole_lines and row_bytes < LONG_ROW_BYTES else LINEAR_F32_LONG_ROW_TILES
+        table = LINEAR_F32_TILES if whole_lines and row_bytes <= F32_ROW_BYTES else LINEAR_F32_OTHER_TILES
     elif gated and whole_lines and row_bytes >= GATED_ROW_BYTES:
         table = LINEAR_GATED_TILES if row_bytes < GATED_LONG_ROW_BYTES else LINEAR_GATED_LONG_ROW_TILES
     elif row_bytes >= LONG_ROW_BYTES and whole_lines and not gated:

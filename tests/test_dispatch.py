@@ -44,7 +44,8 @@ def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
     (256 * 49, 768, 1600, False, False, True, 12), (256 * 101, 768, 768, False, False, True, 13),        # long rows
     (256 * 9, 704, 512, False, False, True, 3), (256 * 101, 512, 512, True, False, False, 11), (256 * 20, 512, 512, True, False, False, 12),
     (256 * 101, 704, 512, True, False, False, 4), (256 * 101, 256, 512, True, False, False, 0), (256 * 20, 256, 512, True, False, False, 6),
-    (256 * 9, 512, 512, False, True, False, 1), (256 * 10, 512, 512, False, True, False, 12), (256 * 10, 768, 768, False, True, False, 7),
+    (256 * 9, 512, 512, False, True, False, 1), (256 * 10, 512, 512, False, True, False, 12), (256 * 10, 768, 768, False, True, False, 12),
+    (256 * 10, 1088, 768, False, True, False, 7),
     (256 * 10, 32, 512, False, True, False, 7),                                                          # rows of no whole lines
     (256 * 10, 96, 512, True, False, False, 6), (256 * 20, 544, 512, True, False, False, 6), (256 * 101, 96, 512, True, False, False, 0)])
 def test_linear_picks_its_tile_by_rows_depth_and_epilogue(monkeypatch, M, K, N, gated, f32, bias, expected):
