@@ -60,9 +60,12 @@ F32_ROW_BYTES = 2048
 # whole L2 lines a step (2,048 inputs: 190 against 226 us at 71,680 rows, 94 against 101 with tile 12 at 35,840; 768 inputs to
 # 768: 79.2 against 91.9 with tile 11 at 49,000); 128 x 64 with 128-byte stages up to 100 rows a compute unit (2,048 inputs at
 # 17,920 rows 54.7 against 58.2 us, 768 inputs 36.8 against 38.6 with tile 11; batch 64 22.0 against 23.8) and 64 x 64 up to 9
-# (batch 16: 11.8 against 20.7 us)
+# (batch 16: 11.8 against 20.7 us). Rows shorter than 2 KB leave 64 x 64 for 128 x 64 (tile 3) from 5 rows a compute unit once it
+# would be more than SMALL_TILES_A_UNIT workgroups a compute unit (768 inputs, with bias: to 1,152 at 1,792 rows, 504 of them,
+# 9.8 and 9.0 us; to 1,600 at 2,048, 800, 14.4 and 12.7; to 768 at 2,048, 384, 8.4 and 8.4; at 1,500, 288, 7.3 and 8.0)
 LINEAR_LONG_ROW_TILES = {"gfx950": [(9, 1), (100, 12), (math.inf, 13)]}
-LONG_ROW_BYTES = 1536
+LINEAR_MANY_TILES = {"gfx950": [(5, 1), (9, 3), (100, 12), (math.inf, 13)]}
+LONG_ROW_BYTES, MANY_TILES_ROW_BYTES, SMALL_TILES_A_UNIT = 1536, 2048, 1.6
 # from this many (position, key/value group) pairs groups_per_workgroup plans a launch of 65 to 80 tokens, query and value
 # widths up to 64, for workgroups of four wavefronts instead of five. (Such launches, and those of 64 tokens, share their pairs
 # out by themselves and only check that the run divides them: csrc/attention_wave.h.)
@@ -81,7 +84,7 @@ def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: b
     return tile != RESIDENT_TILE or (K == RESIDENT_DEPTH and N % 8 == 0 and not gated and bias and not mix and not accumulate_fp32)
 
 
-def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False) -> int:
+def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False, N: int = 0) -> int:
     arch, units = gpu(device)
     whole_lines = row_bytes > 0 and row_bytes % 128 == 0   # (0: the rows' length is not known)
     if accumulate_fp32:
@@ -89,7 +92,8 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
     elif gated and whole_lines and row_bytes >= GATED_ROW_BYTES:
         table = LINEAR_GATED_TILES if row_bytes < GATED_LONG_ROW_BYTES else LINEAR_GATED_LONG_ROW_TILES
     elif row_bytes >= LONG_ROW_BYTES and whole_lines and not gated:
-        table = LINEAR_LONG_ROW_TILES
+        many = row_bytes < MANY_TILES_ROW_BYTES and (M + 63) // 64 * ((N + 63) // 64) > SMALL_TILES_A_UNIT * units
+        table = LINEAR_MANY_TILES if many else LINEAR_LONG_ROW_TILES
     else:
         table = LINEAR_TILES
     return tile_for(table.get(arch, table["gfx950"]), M, units)
@@ -241,7 +245,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
            input_scale: torch.Tensor | None = None) -> torch.Tensor:
     K, width = weight.shape
     M, N = x.numel() // K, width // 2 if gated else width
-    tile = linear_tile(x.device, M, accumulate_fp32, K * x.element_size(), gated)
+    tile = linear_tile(x.device, M, accumulate_fp32, K * x.element_size(), gated, N)
     takes = lambda tile: linear_takes(tile, K, N, gated, bias is not None, residual is not None, accumulate_fp32, original is not None)
     if N in RESIDENT_WIDE_COLUMNS and M > RESIDENT_WIDE_SHARE * gpu(x.device)[1] and takes(RESIDENT_TILE):
         tile = RESIDENT_TILE

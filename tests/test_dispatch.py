@@ -42,6 +42,7 @@ def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
     (256 * 49, 512, 1016, False, False, True, 11), (256 * 49, 512, 1024, False, False, True, 15),        # and least columns
     (256 * 49, 512, 1604, False, False, True, 11), (256 * 49, 512, 1600, False, False, False, 11),       # no whole 8 columns; no bias
     (256 * 49, 768, 1600, False, False, True, 12), (256 * 101, 768, 768, False, False, True, 13),        # long rows
+    (256 * 7, 768, 1152, False, False, True, 3), (256 * 7, 768, 768, False, False, True, 1), (256 * 7, 1024, 1152, False, False, True, 1),
     (256 * 9, 704, 512, False, False, True, 3), (256 * 101, 512, 512, True, False, False, 11), (256 * 20, 512, 512, True, False, False, 12),
     (256 * 101, 704, 512, True, False, False, 4), (256 * 101, 256, 512, True, False, False, 0), (256 * 20, 256, 512, True, False, False, 6),
     (256 * 9, 512, 512, False, True, False, 1), (256 * 10, 512, 512, False, True, False, 12), (256 * 10, 768, 768, False, True, False, 12),
