@@ -35,6 +35,7 @@ LINEAR_TILES = {"gfx950": [(5, 1), (9, 3), (48, 6), (100, 11), (math.inf, 15)]}
 # projection to 1,600 columns: 155.7 against 200.2 us on tile 0); other linears of the table's share take tile 0, the
 # kernel's own pick by size
 RESIDENT_TILE, RESIDENT_DEPTH = 15, 512
+RESIDENT_OUTPUT_BYTES, RESIDENT_COLUMNS = 1 << 31, 32 * 256   # its outputs' (32-bit offsets) and its column groups' limits
 # and from this share on where it has 1,024 columns or more, so that each of its workgroups still has a long stream of row
 # blocks (512 to 1,600 columns at 17,920 rows, graphs of launches: 37.4 against 43.0 us on tile 11); up to 4,096, inside the
 # column groups and output bytes it takes
@@ -78,10 +79,12 @@ def tile_for(tiles: list[tuple[float, object]], M: int, multiprocessors: int):
     return next(tile for most, tile in tiles if share <= most)
 
 
-def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: bool, accumulate_fp32: bool, mix: bool = False) -> bool:
+def linear_takes(tile: int, K: int, N: int, gated: bool, bias: bool, residual: bool, accumulate_fp32: bool, mix: bool = False, M: int = 0) -> bool:
     """Whether linear's tile takes the launch: every tile does but 15, which takes fp16 sums of depth 512 into N a multiple of
-    8 with the bias (and the residual or not), not gated, without the next block's input mix, in fp16."""
-    return tile != RESIDENT_TILE or (K == RESIDENT_DEPTH and N % 8 == 0 and not gated and bias and not mix and not accumulate_fp32)
+    8, at most 8,192, with the bias (and the residual or not), not gated, without the next block's input mix, in fp16, and M rows
+    (where given) of less than 2 GiB."""
+    return tile != RESIDENT_TILE or (K == RESIDENT_DEPTH and N % 8 == 0 and N <= RESIDENT_COLUMNS and 2 * M * N < RESIDENT_OUTPUT_BYTES
+                                     and not gated and bias and not mix and not accumulate_fp32)
 
 
 def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row_bytes: int = 0, gated: bool = False, N: int = 0) -> int:
@@ -246,7 +249,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     K, width = weight.shape
     M, N = x.numel() // K, width // 2 if gated else width
     tile = linear_tile(x.device, M, accumulate_fp32, K * x.element_size(), gated, N)
-    takes = lambda tile: linear_takes(tile, K, N, gated, bias is not None, residual is not None, accumulate_fp32, original is not None)
+    takes = lambda tile: linear_takes(tile, K, N, gated, bias is not None, residual is not None, accumulate_fp32, original is not None, M)
     if N in RESIDENT_WIDE_COLUMNS and M > RESIDENT_WIDE_SHARE * gpu(x.device)[1] and takes(RESIDENT_TILE):
         tile = RESIDENT_TILE
     elif not takes(tile):

@@ -69,6 +69,9 @@ SPLIT_WAVES = {14: 4}
 # multiple of 128, not gated, no bias, the residual added (with or without the next block's mix)
 RESIDENT_TILE, RESIDENT_DEPTH = 15, 512
 DEEP_TILE, DEEP_DEPTH = 16, 2048
+# and their launches' limits: outputs under 2 GiB (32-bit offsets of two-byte values), and no more column groups (of 256 gated
+# and 512 other columns, and of 128) than the compute units of an XCD
+RESIDENT_OUTPUT_BYTES, RESIDENT_GROUPS = 1 << 31, 32
 # each tile's (rows, output columns, wavefronts, ring stages), the shapes the kernels are instantiated with
 TILE_SHAPES = {1: (64, 64, 4, 4), 2: (128, 128, 4, 4), 3: (128, 64, 4, 4), 4: (256, 128, 8, 3), 5: (128, 128, 8, 2), 6: (128, 128, 8, 3),
                7: (128, 128, 4, 3), 8: (128, 64, 4, 3), 9: (128, 64, 4, 2), 10: (256, 64, 4, 2), 11: (128, 128, 4, 2), 12: (128, 64, 4, 2),
@@ -125,13 +128,15 @@ def gpu_arch(device: torch.device) -> str:
     return torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
 
 
-def tile_takes(tile: int, N: int, K: int, gated: bool = False, bias: bool = False, residual: bool = False) -> bool:
-    """Whether tile takes N outputs of depth K with that epilogue; the whole-K tiles take every shape int8_linear takes, the
-    split-K and register-held ones only some."""
+def tile_takes(tile: int, N: int, K: int, gated: bool = False, bias: bool = False, residual: bool = False, M: int = 0) -> bool:
+    """Whether tile takes N outputs of depth K with that epilogue (of M rows, where given); the whole-K tiles take every shape
+    int8_linear takes, the split-K and register-held ones only some."""
+    if tile in (RESIDENT_TILE, DEEP_TILE) and 2 * M * N >= RESIDENT_OUTPUT_BYTES:
+        return False
     if tile == RESIDENT_TILE:
-        return K == RESIDENT_DEPTH and N % 8 == 0 and not residual
+        return K == RESIDENT_DEPTH and N % 8 == 0 and not residual and N <= RESIDENT_GROUPS * (256 if gated else 512)
     if tile == DEEP_TILE:
-        return K == DEEP_DEPTH and N % 128 == 0 and not gated and not bias and residual
+        return K == DEEP_DEPTH and N % 128 == 0 and not gated and not bias and residual and N <= RESIDENT_GROUPS * 128
     waves = SPLIT_WAVES.get(tile)
     return waves is None or (N % 8 == 0 and K % (128 * waves) == 0 and K // (128 * waves) in (1, 2, 4))
 
@@ -150,7 +155,7 @@ def int8_tile(device: torch.device, matmul: str, M: int, N: int = 0, K: int = 0,
     candidates = [tile for most, tile in tiles if share <= most]
     gated = matmul == "gate_up" if gated is None else gated
     residual = matmul == "down" if residual is None else residual
-    return next((tile for tile in candidates if not N or tile_takes(tile, N, K, gated, bias, residual)), 0)
+    return next((tile for tile in candidates if not N or tile_takes(tile, N, K, gated, bias, residual, M)), 0)
 
 
 def config_for(device: torch.device, kind: str, M: int, K: int, N: int = 0) -> int:

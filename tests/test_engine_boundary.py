@@ -161,3 +161,25 @@ def test_the_register_held_tiles_take_only_their_launches():
     assert not any((linear_takes(15, 512, 512, False, True, True, False, True), linear_takes(15, 512, 512, True, True, False, False),
                     linear_takes(15, 512, 512, False, False, True, False), linear_takes(15, 512, 512, False, True, True, True)))
     assert linear_takes(11, 2048, 512, True, False, True, True, True)
+
+
+def test_launches_past_the_register_held_tiles_limits_take_tile_0(monkeypatch):
+    """Tiles 15 and 16 write outputs under 2 GiB and take at most 32 column groups (a compute unit's XCD has 32 on an MI355X); the
+    tables' and linear's choices give larger launches to tile 0, which takes them (8,192 positions of the d512 network: gate_up
+    writes 2.3 GB)."""
+    from model import fused_blocks, hip_kernels
+    monkeypatch.setattr(hip_kernels, "gpu", lambda device: ("gfx950", 256))
+    monkeypatch.setattr(fused_blocks, "gpu", lambda device: ("gfx950", 256))
+    cuda, chosen = torch.device("cuda"), []
+    tile = int8_blocks.int8_tile
+    assert [tile(cuda, "gate_up", positions * 70, 2048, 512) for positions in (7489, 7490, 8192)] == [15, 0, 0]
+    assert tile(cuda, "gate_up", 524287, 2048, 512) == 15 and tile(cuda, "gate_up", 524288, 2048, 512) == 0
+    assert tile(cuda, "projection", 671088, 1600, 512, bias=True) == 15 and tile(cuda, "projection", 671089, 1600, 512, bias=True) == 0
+    assert tile(cuda, "down", 2097151, 512, 2048) == 16 and tile(cuda, "down", 2097152, 512, 2048) == 0
+    assert tile(cuda, "gate_up", 71680, 8192, 512) == 15 and tile(cuda, "gate_up", 71680, 8200, 512) == 0
+    assert tile(cuda, "down", 71680, 4096, 2048) == 16 and tile(cuda, "down", 71680, 4224, 2048) == 0
+    monkeypatch.setattr(fused_blocks, "launch_linear", lambda x, weight, *arguments: chosen.append(arguments[-1]) or x.new_empty(0))
+    for M, N in ((262143, 4096), (262144, 4096), (71680, 8192), (71680, 8200)):
+        x = torch.empty(1, dtype=torch.float16).expand(M, 512)
+        fused_blocks.linear(x, torch.empty(1, dtype=torch.float16).expand(512, N), torch.empty(1, dtype=torch.float16).expand(N))
+    assert chosen == [15, 0, 15, 0]

@@ -899,3 +899,17 @@ def test_the_kernels_run_in_graphs_on_two_streams(device):
         torch.cuda.synchronize()
         for found, answer in zip(outputs, expected):
             assert all(torch.equal(a, b) for a, b in zip(found, answer)), replay
+
+
+def test_outputs_of_two_gib_take_the_kernels_own_pick(device):
+    """524,304 rows of 512 to 2 x 2,048 columns write 2 GiB, past what tile 15's 32-bit offsets take: the table's choice gives
+    them to tile 0, whose first and last rows are a small launch's bits."""
+    M, ends = 524304, 48
+    x, x_scale, weight, weight_scale, bias, residual, gated, mix = int8_operands("gate_up", ends, device, width=2048, depth=512)
+    many = torch.zeros(M, 512, device=device, dtype=torch.int8)
+    scales = torch.ones(M, device=device)
+    for at in (slice(0, ends), slice(M - ends, M)):
+        many[at], scales[at] = x, x_scale
+    out = int8_linear(many, scales, weight, weight_scale, None, None, True, "gate_up")
+    expected = launch_int8_linear(x, x_scale, weight, weight_scale, None, None, True, None, None, None, 1)
+    assert same_bits(out[:ends], expected) and same_bits(out[-ends:], expected) and not out[ends:-ends].any()
