@@ -59,9 +59,9 @@ INT8_TILES = {"gfx950": {"projection": [(0.55, 14), (5, 1), (9, 8), (100, 11), (
 # projection of rows longer than 512 (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 7.9 us on tile 6 and
 # 9.0 on tile 11, 7,000 in 11.3 on tile 13 and 12.7, 17,920 in 25.2 and 27.8; past them tile 0, which takes the weights in
 # registers at such depths too (35,000 rows: 40.7 against 47.1 us on tile 13, 69,930 75.1 against 98.2)
-# (for the shipped table only: one put in INT8_TILES in its place holds for every depth)
+# (for the shipped table only: one put in INT8_TILES in its place, or edited there, holds for every depth)
 LONG_PROJECTION_TILES = {"gfx950": [(0.55, 14), (5, 1), (9, 8), (20, 6), (75, 13), (math.inf, 0)]}
-SHIPPED_PROJECTION_TILES = INT8_TILES["gfx950"]["projection"]
+SHIPPED_PROJECTION_TILES = list(INT8_TILES["gfx950"]["projection"])
 # the split-K tile's wavefronts: each reads 1, 2 or 4 steps of 128 bytes of K, and the outputs go 8 columns a lane
 SPLIT_WAVES = {14: 4}
 # the tiles whose wavefronts hold their weights in registers for the whole depth: 15 (gemm_resident.h) at depth 512, N a
@@ -149,7 +149,7 @@ def int8_tile(device: torch.device, matmul: str, M: int, N: int = 0, K: int = 0,
     takes them: 0, the kernel's own pick of a whole-K tile, which takes every shape)."""
     arch, units = hip_kernels.gpu(device)
     tiles = INT8_TILES.get(arch, INT8_TILES["gfx950"])[matmul]
-    if tiles is SHIPPED_PROJECTION_TILES and K > RESIDENT_DEPTH and K % 128 == 0:
+    if matmul == "projection" and tiles == SHIPPED_PROJECTION_TILES and K > RESIDENT_DEPTH and K % 128 == 0:
         tiles = LONG_PROJECTION_TILES.get(arch, LONG_PROJECTION_TILES["gfx950"])
     share = M / units
     candidates = [tile for most, tile in tiles if share <= most]

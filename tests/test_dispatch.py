@@ -24,6 +24,10 @@ def test_a_projection_table_put_in_the_shipped_ones_place_holds_at_every_depth(m
     assert (chosen(512), chosen(768), chosen(832)) == (11, 6, 11)   # 832: no whole 128-byte lines
     monkeypatch.setitem(int8_blocks.INT8_TILES["gfx950"], "projection", [(math.inf, 3)])
     assert (chosen(512), chosen(768)) == (3, 3)
+    monkeypatch.setitem(int8_blocks.INT8_TILES["gfx950"], "projection", list(int8_blocks.SHIPPED_PROJECTION_TILES))   # put back
+    assert (chosen(512), chosen(768), chosen(832)) == (11, 6, 11)
+    int8_blocks.INT8_TILES["gfx950"]["projection"][-2] = (100, 2)                                                    # edited in place
+    assert (chosen(512), chosen(768)) == (2, 2)
 
 
 def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
