@@ -124,10 +124,6 @@ def apply_overrides(environment=os.environ) -> None:
 apply_overrides()
 
 
-def gpu_arch(device: torch.device) -> str:
-    return torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
-
-
 def tile_takes(tile: int, N: int, K: int, gated: bool = False, bias: bool = False, residual: bool = False, M: int = 0) -> bool:
     """Whether tile takes N outputs of depth K with that epilogue (of M rows, where given); the whole-K tiles take every shape
     int8_linear takes, the split-K and register-held ones only some."""
@@ -186,8 +182,9 @@ def rotated_down_tile(device: torch.device, M: int, hidden: int, width: int) -> 
     as two launches). The folded kernel takes no padding columns and whole blocks of 128."""
     if hidden != width or width % 128 or M == 0:
         return 0
-    shares = ROTATED_DOWN_TILES.get(gpu_arch(device), [(math.inf, 0)])
-    share = M / torch.cuda.get_device_properties(device).multi_processor_count
+    arch, units = hip_kernels.gpu(device)
+    shares = ROTATED_DOWN_TILES.get(arch, [(math.inf, 0)])
+    share = M / units
     return next(tile for most, tile in shares if share <= most)
 
 

@@ -41,6 +41,23 @@ def test_the_tile_choices_ask_torch_about_what_is_no_gpu(monkeypatch):
             hip_kernels.gpu(device)
 
 
+def test_no_choice_of_an_int8_block_asks_torch_for_its_properties(monkeypatch):
+    """A block's choices of tiles and rows ask for the GPU's target and compute units through hip_kernels.gpu, which asks torch once
+    a process."""
+    def properties(device):
+        raise AssertionError("torch was asked")
+    monkeypatch.setattr(torch.cuda, "get_device_properties", properties)
+    monkeypatch.setattr(hip_kernels, "_gpus", {0: ("gfx950", 256)})
+    device = torch.device("cuda", 0)
+    for M in (70, 4480, 71680):
+        int8_blocks.rotate_rows(device, M)
+        int8_blocks.rotated_down_tile(device, M, 2048, 2048)
+        for role in ("projection", "gate_up", "down"):
+            int8_blocks.int8_tile(device, role, M, 512, 512)
+        for f32, gated in ((False, False), (False, True), (True, False)):
+            fused_blocks.linear_tile(device, M, f32, 1024, gated, 512)
+
+
 @pytest.mark.parametrize("M, K, N, gated, f32, bias, expected", [
     (256 * 48, 512, 1600, False, False, True, 6), (256 * 48 + 1, 512, 1600, False, False, True, 15),    # the long streams' first row
     (256 * 49, 512, 1016, False, False, True, 11), (256 * 49, 512, 1024, False, False, True, 15),        # and least columns
