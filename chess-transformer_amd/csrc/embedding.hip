@@ -33,7 +33,8 @@ struct Codes {
 constexpr int TOKENS_A_GROUP = 8;
 constexpr int THREADS = 256;
 
-template <typename Code>
+// Place: what holds a row's place in the table, in 16-byte chunks: 32 bits, or 64 for tables of 64 GiB or more
+template <typename Code, typename Place>
 __global__ __launch_bounds__(THREADS) void board_embedding_kernel(
     const Code* __restrict__ boards, const int* __restrict__ rays, const int* __restrict__ jumps, const int* __restrict__ offsets,
     const half_t* __restrict__ embed, const half_t* __restrict__ position, const half_t* __restrict__ table, half_t* __restrict__ out,
@@ -42,7 +43,7 @@ __global__ __launch_bounds__(THREADS) void board_embedding_kernel(
     __shared__ int square_codes[SQUARES + 1];     // the 65th is the code past the edge
     __shared__ int token_codes[TOKENS_A_GROUP];
     __shared__ int first[4];
-    __shared__ __align__(16) uint32_t rows[TOKENS_A_GROUP][FEATURES + 1];   // each row's place in the table, in 16-byte chunks
+    __shared__ __align__(16) Place rows[TOKENS_A_GROUP][FEATURES + 1];
 
     const int tid = threadIdx.x;
     const int groups = (T + TOKENS_A_GROUP - 1) / TOKENS_A_GROUP, chunks = D / 8;
@@ -72,10 +73,10 @@ __global__ __launch_bounds__(THREADS) void board_embedding_kernel(
     // thread also the kings' and queens' places and the knights, which it counts over the square's eight threads
     const int jump_code = square_codes[min(max(jump, 0), SQUARES)];
     const uint64_t ours_at = __ballot(finds && jump_code == codes.knight), theirs_at = __ballot(finds && jump_code == codes.knight + codes.theirs);
-    auto place = [&](int row) { return (uint32_t)min(max(row, 0), table_rows - 1) * (uint32_t)chunks; };
+    auto place = [&](int row) { return (Place)min(max(row, 0), table_rows - 1) * (Place)chunks; };
     if (finds) {
         const int file = s % 8, rank = s / 8;
-        uint32_t* row = rows[local];
+        Place* row = rows[local];
         const int steps[STEPS] = {near[0], near[1], near[2], near[3], far[0], far[1], far[2], far[3]};
         const int pawn_theirs = codes.pawn + codes.theirs;
         int line = 0, pawn = 0;
@@ -153,11 +154,12 @@ extern "C" int chess_board_embedding(const void* boards, int code_bytes, const v
     if (!aligned16(embed) || !aligned16(position) || !aligned16(table) || !aligned16(out))
         return chess_fail(CHESS_MISALIGNED, "board_embedding's 16-byte loads need aligned tables and output");
     const Codes codes{pawn, knight, queen, king, theirs, edge, no_piece};
-    if ((uint64_t)table_rows * (D / 8) >= (1ull << 32)) return chess_fail(CHESS_UNSUPPORTED, "board_embedding takes tables under 64 GiB");
     const long grid = (long)B * ((T + TOKENS_A_GROUP - 1) / TOKENS_A_GROUP);
+    const bool wide = (uint64_t)table_rows * (D / 8) >= (1ull << 32);
     auto launch = [&](auto code) {
         typedef decltype(code) Code;
-        hipLaunchKernelGGL(board_embedding_kernel<Code>, dim3(grid), dim3(THREADS), 0, (hipStream_t)stream, (const Code*)boards,
+        auto kernel = wide ? board_embedding_kernel<Code, uint64_t> : board_embedding_kernel<Code, uint32_t>;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(THREADS), 0, (hipStream_t)stream, (const Code*)boards,
                            (const int*)rays, (const int*)jumps, (const int*)offsets, (const half_t*)embed, (const half_t*)position,
                            (const half_t*)table, (half_t*)out, T, D, embed_rows, table_rows, codes);
     };

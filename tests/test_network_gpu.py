@@ -368,3 +368,24 @@ def test_the_board_embedding_is_the_oracles_to_the_bit(device, d_model, codes):
     out = embedding(boards.to(device, codes))
     expected = oracle_network.input_embedding(boards.numpy(), state["embed.weight"], state["position_embed"], state["square_features.table"])
     assert out.dtype == torch.float16 and torch.equal(out.cpu(), torch.from_numpy(expected))
+
+
+def test_the_board_embedding_reads_tables_past_64_gib(device):
+    """A table of 2^32 16-byte chunks and more, whose rows past that place are a small table's: the small table's bits."""
+    if torch.cuda.mem_get_info(device)[0] < 100 << 30:
+        pytest.skip("the table takes 64 GiB of the GPU's memory")
+    D = 32768
+    model = ChessTransformer(d_model=64, num_layers=1, n_heads=4).eval()
+    embedding = fused_blocks.InputEmbedding(model.half()).to(device)
+    generator = torch.Generator(device=device).manual_seed(7)
+    rows = len(model.square_features.table)
+    embed, position, table = (torch.randn(count, D, device=device, generator=generator).half() for count in (len(model.embed.weight), 70, rows))
+    boards = random_boards(3, seed=9).to(device)
+    expected = fused_blocks.board_embedding(boards, embedding.rays, embedding.jumps, embedding.offsets, embed, position, table)
+    first = (1 << 32) // (D // 8)
+    large = torch.empty(first + rows, D, device=device, dtype=torch.float16)
+    large[first:] = table
+    out = fused_blocks.board_embedding(boards, embedding.rays, embedding.jumps, embedding.offsets + first, embed, position, large)
+    del large
+    torch.cuda.empty_cache()
+    assert torch.equal(out, expected)
