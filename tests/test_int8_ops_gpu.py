@@ -701,28 +701,43 @@ def test_template_attention_reads_the_templates_and_their_coefficients(device):
     assert (template_attention(projected, templates, *rest).float() - without_bias.float()).abs().max() > 0.05
 
 
-def test_groups_a_workgroup_change_no_bit(device):
-    """Any run of (position, key/value group) pairs a workgroup takes gives the same bits, runs across positions too (12: three
-    positions' 4 groups each; 36: all nine positions in one workgroup)."""
-    arguments = attention_operands(device, 9, 8, 4, 32, 32, seed=3)
-    found = [launch_template_attention(*arguments, groups_per_block=groups) for groups in (1, 2, 4, 3, 12, 36)]
-    assert all(torch.equal(found[0], other) for other in found[1:])
+@pytest.mark.parametrize("heads, kv_heads, dq, dv, tokens, count, dtype", [
+    (8, 4, 32, 32, 100, 8, torch.float16), (8, 4, 32, 32, 100, 6, torch.bfloat16), (8, 4, 64, 64, 128, 8, torch.float16),
+    (8, 8, 64, 64, 128, 8, torch.bfloat16), (4, 4, 64, 128, 70, 8, torch.float16), (6, 3, 24, 128, 96, 8, torch.float16),
+    (4, 4, 128, 64, 70, 8, torch.float16), (2, 2, 104, 128, 80, 8, torch.float16)])
+def test_groups_a_workgroup_change_no_bit(device, heads, kv_heads, dq, dv, tokens, count, dtype):
+    """Any run of (position, key/value group) pairs a workgroup takes gives the same bits, and the fp32 formula's answer, runs
+    across positions and all nine positions in one workgroup too: the kernel of more than 80 tokens or widths past 64, which walks
+    the runs through two buffers, its outputs staged over the queries (value widths up to the queries') or stored from the
+    registers. (The other kernel shares the pairs out by itself.)"""
+    projected, *rest = attention_operands(device, 9, heads, kv_heads, dq, dv, seed=tokens + dv, tokens=tokens, templates_count=count)
+    arguments, pairs = (projected.to(dtype), *rest), 9 * kv_heads
+    one = launch_template_attention(*arguments, groups_per_block=1)
+    assert (one.float() - reference_attention(arguments)).abs().max() < 1e-2
+    for groups in [groups for groups in range(2, pairs + 1) if pairs % groups == 0]:
+        assert torch.equal(launch_template_attention(*arguments, groups_per_block=groups), one), groups
     with pytest.raises(ValueError):
-        launch_template_attention(*arguments, groups_per_block=5)   # not a divisor of the 36 pairs
+        launch_template_attention(*arguments, groups_per_block=5)   # not a divisor of the pairs
+
+
+def whole_pair_positions(device, kv_heads, dq, dv):
+    """A few positions more than the most that the kernel of widths up to 64 shares over four wavefronts a pair (65 to 80 tokens)."""
+    units = torch.cuda.get_device_properties(device).multi_processor_count
+    return (6 if dq <= 32 and dv <= 32 else 4) * units // kv_heads + 5
 
 
 @pytest.mark.parametrize("heads, kv_heads, dq, dv, tokens", [(8, 8, 64, 64, 70), (8, 4, 32, 32, 80), (4, 4, 16, 64, 65), (6, 3, 64, 16, 66)])
-def test_the_split_slab_launch_gives_the_small_launchs_bits(device, heads, kv_heads, dq, dv, tokens):
-    """65 to 80 tokens: from ATTENTION_SPLIT_PAIRS (position, key/value group) pairs a launch splits the slab past the squares over three
-    wavefronts; every position's rows are the same bits as in launches of seven positions (unsplit), and the answer is the
-    fp32 formula's. The grouped case with two heads a group (6 on 3) once differed on the tokens past the squares of a few
-    positions in the middle of the launch."""
-    positions = -(-fused_blocks.ATTENTION_SPLIT_PAIRS // kv_heads) + 5
+def test_large_attention_launches_give_the_small_launchs_bits(device, heads, kv_heads, dq, dv, tokens):
+    """65 to 80 tokens: in a large launch a wavefront takes whole (position, key/value group) pairs; every position's rows are the
+    same bits as in launches of seven positions (four wavefronts a pair), and the answer is the fp32 formula's. The grouped case
+    with two heads a group (6 on 3) once differed on the tokens past the squares of a few positions in the middle of the
+    launch."""
+    positions = whole_pair_positions(device, kv_heads, dq, dv)
     arguments = attention_operands(device, positions, heads, kv_heads, dq, dv, seed=tokens, tokens=tokens)
-    split = template_attention(*arguments)
-    assert torch.allclose(split.float(), reference_attention(arguments), atol=1e-2)
+    large = template_attention(*arguments)
+    assert torch.allclose(large.float(), reference_attention(arguments), atol=1e-2)
     few = torch.cat([template_attention(arguments[0][start:start + 7].contiguous(), *arguments[1:]) for start in range(0, positions, 7)])
-    assert torch.equal(few, split)
+    assert torch.equal(few, large)
 
 
 @pytest.mark.parametrize("heads, kv_heads, dq, dv, tokens, count, positions", [
@@ -812,14 +827,14 @@ def test_bf16_template_attention_at_64_tokens_with_a_bias_per_head(device, posit
     assert (out.float() - reference_attention(arguments)).abs().max() < 1e-2
 
 
-def test_bf16_split_slab_launch_gives_the_small_launchs_bits(device):
-    """bf16 rows at 70 tokens from ATTENTION_SPLIT_PAIRS pairs (the split slab): a position's rows are a three-position launch's bits."""
-    positions = fused_blocks.ATTENTION_SPLIT_PAIRS // 8
+def test_large_bf16_attention_launches_give_the_small_launchs_bits(device):
+    """bf16 rows at 70 tokens, a wavefront a pair: a position's rows are a three-position launch's bits."""
+    positions = whole_pair_positions(device, 8, 64, 64)
     arguments = bf16_operands(attention_operands(device, positions, 8, 8, 64, 64, seed=70, tokens=70))
-    split = template_attention(*arguments)
-    assert (split.float() - reference_attention(arguments)).abs().max() < 1e-2
+    large = template_attention(*arguments)
+    assert (large.float() - reference_attention(arguments)).abs().max() < 1e-2
     for rows in (slice(0, 3), slice(positions - 3, positions)):
-        assert torch.equal(template_attention(arguments[0][rows].contiguous(), *arguments[1:]), split[rows]), rows
+        assert torch.equal(template_attention(arguments[0][rows].contiguous(), *arguments[1:]), large[rows]), rows
 
 
 def test_template_attention_refuses_what_it_cannot_take(device):
