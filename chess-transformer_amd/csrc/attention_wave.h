@@ -11,7 +11,7 @@
 //           normalising the keys for itself; the templates come from global memory. The shorter chain, for small launches.
 // Timed on an MI355X, as the launches of a graph (us, before and after): 70 tokens, 8 x 64 heads: batch 1024 98.6 and 67.1,
 // 256 31.3 and 21.6, 64 13.1 and 11.0, 1 8.3 and 7.5; 24 on 12 heads, query width 16, value width 32: batch 700 201 and 80, 51
-// 26.9 and 14.3; 8 x 32 heads: batch 999 84 and 41; 64 tokens, 8 x 64 heads in bf16: batch 4096 283 and 264. Bound by its VALU
+// 26.9 and 14.3; 8 x 32 heads: batch 999 84 and 41; 64 tokens, 8 x 64 heads in bf16: batch 4096 264 and 231. Bound by its VALU
 // work beside waits that two wavefronts a SIMD do not cover: at batch 1024 the VALU is busy for half of the kernel's cycles;
 // the rows alone would take 44 us at the rate of a large copy.
 #pragma once
@@ -206,7 +206,7 @@ void template_attention_wave_kernel(
             else buffer_dma16(rows, (LDS_SPACE void*)(values + i * 1024), lane_at, at + row_at);
         }
     };
-    // the templates of the wavefront's own slab, in the steps' order (FOURS and SLABS)
+    // the templates of the wavefront's own slab, in the steps' order (FOURS)
     v4u slab_templates[MODE == WHOLE ? 1 : 4][4];
     auto load_templates = [&] {
         if constexpr (MODE != WHOLE) {
@@ -234,7 +234,7 @@ void template_attention_wave_kernel(
         return uint2{two_halves(bias[0], bias[1]), two_halves(bias[2], bias[3])};
     };
     uint2 slab_bias[4];
-    auto take_slab_bias = [&] {   // the wavefront's own slab's (FOURS and SLABS)
+    auto take_slab_bias = [&] {   // the wavefront's own slab's (FOURS)
         if constexpr (MODE != WHOLE) {
             v8h mix[4];
             coefficients(mix);

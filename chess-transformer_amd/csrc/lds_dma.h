@@ -40,10 +40,6 @@ DEVICE uint4 buffer_load16(BufferResource resource, uint32_t lane_offset, uint32
     const v4u v = __builtin_amdgcn_raw_buffer_load_b128(resource, lane_offset, offset, 0);
     return uint4{v[0], v[1], v[2], v[3]};
 }
-DEVICE uint4 buffer_load16_streamed(BufferResource resource, uint32_t lane_offset, uint32_t offset) {   // non-temporal
-    const v4u v = __builtin_amdgcn_raw_buffer_load_b128(resource, lane_offset, offset, 2);
-    return uint4{v[0], v[1], v[2], v[3]};
-}
 // 8 and 4 bytes a lane from a buffer into registers (zeros past the resource's bytes)
 DEVICE uint2 buffer_load8(BufferResource resource, uint32_t lane_offset, uint32_t offset) {
     const v2u v = __builtin_amdgcn_raw_buffer_load_b64(resource, lane_offset, offset, 0);
@@ -73,7 +69,6 @@ DEVICE void buffer_dma16(BufferResource, LDS_SPACE void*, uint32_t, uint32_t) {}
 DEVICE void buffer_dma4(BufferResource, LDS_SPACE void*, uint32_t, uint32_t) {}
 DEVICE void buffer_dma16_streamed(BufferResource, LDS_SPACE void*, uint32_t, uint32_t) {}
 DEVICE uint4 buffer_load16(BufferResource, uint32_t, uint32_t) { return uint4{0, 0, 0, 0}; }
-DEVICE uint4 buffer_load16_streamed(BufferResource, uint32_t, uint32_t) { return uint4{0, 0, 0, 0}; }
 DEVICE uint2 buffer_load8(BufferResource, uint32_t, uint32_t) { return uint2{0, 0}; }
 DEVICE uint32_t buffer_load4(BufferResource, uint32_t, uint32_t) { return 0; }
 DEVICE void buffer_store8(BufferResource, uint2, uint32_t, uint32_t) {}

@@ -67,10 +67,9 @@ F32_ROW_BYTES = 2048
 LINEAR_LONG_ROW_TILES = {"gfx950": [(9, 1), (100, 12), (math.inf, 13)]}
 LINEAR_MANY_TILES = {"gfx950": [(5, 1), (9, 3), (100, 12), (math.inf, 13)]}
 LONG_ROW_BYTES, MANY_TILES_ROW_BYTES, SMALL_TILES_A_UNIT = 1536, 2048, 1.6
-# from this many (position, key/value group) pairs groups_per_workgroup plans a launch of 65 to 80 tokens, query and value
-# widths up to 64, for workgroups of four wavefronts instead of five. (Such launches, and those of 64 tokens, share their pairs
-# out by themselves and only check that the run divides them: csrc/attention_wave.h.)
-ATTENTION_SPLIT_PAIRS = 1024
+# template_attention launches of up to this many tokens, query and value widths up to this, share their pairs out by themselves
+# (csrc/attention_wave.h) and take any run of pairs a workgroup; the others take groups_per_workgroup's
+ATTENTION_SHARING_TOKENS, ATTENTION_SHARING_WIDTH = 80, 64
 
 
 # tiles lists (share, tile) pairs by growing share; a launch takes the first whose share bounds M / multiprocessors (the last bounds any)
@@ -102,22 +101,18 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
     return tile_for(table.get(arch, table["gfx950"]), M, units)
 
 
-def attention_waves(positions: int, kv_heads: int, tokens: int, dq: int, dv: int) -> int:
-    """The wavefronts that a template_attention workgroup is planned with: one a slab of 16 queries, or four in launches of
-    ATTENTION_SPLIT_PAIRS on, where the fifth slab is one of the four's too."""
-    tiles = (tokens + 15) // 16
-    split = tiles == 5 and dq <= 64 and dv <= 64 and positions * kv_heads >= ATTENTION_SPLIT_PAIRS
-    return 4 if split else tiles
+def attention_waves(tokens: int) -> int:
+    """The wavefronts of a template_attention workgroup that walks a run of pairs: one a slab of 16 queries."""
+    return (tokens + 15) // 16
 
 
-def groups_per_workgroup(positions: int, kv_heads: int, multiprocessors: int = 256, tokens: int = 70, dq: int = 64, dv: int = 64) -> int:
+def groups_per_workgroup(positions: int, kv_heads: int, multiprocessors: int = 256, tokens: int = 70) -> int:
     """The most (position, key/value group) pairs a workgroup takes -- a divisor of all the launch's pairs -- while the launch
     keeps as many workgroups as the compute units hold at once (two wavefronts a SIMD, four SIMDs: one workgroup of five to
     eight wavefronts, two of four), so that a workgroup's start (its template registers and first loads) is paid once for
-    its pairs; any choice gives the same bits. It is what heads wider than 64 and more than 80 tokens run with; the others
-    balance themselves, which no divisor can: 24 on 12 heads at batch 700 had 525 workgroups of 16 pairs for 512 places."""
+    its pairs; any choice gives the same bits."""
     pairs = positions * kv_heads
-    workgroups = multiprocessors * max(1, 8 // attention_waves(positions, kv_heads, tokens, dq, dv))
+    workgroups = multiprocessors * max(1, 8 // attention_waves(tokens))
     groups = max(1, pairs // workgroups)
     while pairs % groups:
         groups -= 1
@@ -143,7 +138,8 @@ def launch_template_attention(projected: torch.Tensor, templates: torch.Tensor, 
     projected = aligned(projected)
     keyed = keyed_templates(templates, templates_count)
     out = torch.empty(B, T, heads * dv, device=projected.device, dtype=projected.dtype)
-    groups = groups_per_block or groups_per_workgroup(B, kv_heads, gpu(projected.device)[1], T, dq, dv)
+    shares = T <= ATTENTION_SHARING_TOKENS and max(dq, dv) <= ATTENTION_SHARING_WIDTH
+    groups = groups_per_block or (1 if shares else groups_per_workgroup(B, kv_heads, gpu(projected.device)[1], T))
     entry = library.chess_template_attention_bf16 if bf16 else library.chess_template_attention
     code = entry(pointer(projected), pointer(keyed), pointer(q_gain.contiguous()), pointer(k_gain.contiguous()), pointer(out), B, T, heads,
                  kv_heads, dq, dv, templates_count, groups, float(eps), 1 / math.sqrt(dq), stream_of(projected.device))

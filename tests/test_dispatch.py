@@ -114,16 +114,14 @@ def test_attention_runs_divide_the_pairs_and_keep_the_chip_busy(positions, kv_he
     # at least one workgroup a compute unit when there are enough pairs; when a workgroup takes several pairs, no more
     # workgroups than the compute units hold at once
     assert workgroups >= min(pairs, 256)
-    assert groups == 1 or workgroups <= 256 * (8 // fused_blocks.attention_waves(positions, kv_heads, tokens, 64, 64)) * 2
+    assert groups == 1 or workgroups <= 256 * (8 // fused_blocks.attention_waves(tokens)) * 2
 
 
-def test_attention_runs_at_the_timed_batches():
-    # batch 16: one pair a workgroup; batch 64: 256 workgroups of 2; batches 128, 256 and 1024 (the split slab, two
-    # workgroups a compute unit): 512 workgroups of 2, 4 and 16
-    assert [groups_per_workgroup(b, 8, 256) for b in (16, 64, 128, 256, 1024)] == [1, 2, 2, 4, 16]
-    assert [fused_blocks.attention_waves(b, 8, 70, 64, 64) for b in (64, 127, 128)] == [5, 5, 4]
-    # the split slab takes 65 to 80 tokens and widths up to 64
-    assert [fused_blocks.attention_waves(1024, 8, t, 64, dv) for t, dv in ((64, 64), (81, 64), (80, 128), (65, 16))] == [4, 6, 5, 4]
+def test_attention_runs_by_tokens():
+    """One workgroup a compute unit at five slabs of 16 tokens and more, two at four (8 key/value groups)."""
+    assert [groups_per_workgroup(b, 8, 256, 100) for b in (16, 64, 128, 256, 1024)] == [1, 2, 4, 8, 32]
+    assert [groups_per_workgroup(b, 8, 256, 64) for b in (16, 64, 128, 256, 1024)] == [1, 1, 2, 4, 16]
+    assert [fused_blocks.attention_waves(tokens) for tokens in (64, 65, 80, 81, 128)] == [4, 5, 5, 6, 8]
 
 
 def test_the_move_tables_are_the_gathers_of_the_heads():
