@@ -502,23 +502,23 @@ template <typename In, int NB, typename OutT, typename F> bool taken(int flags, 
 
 // The least row blocks a workgroup's stream has to hold for the launch to pay for its weights' load and its ends. Timed on an
 // MI355X as graphs of launches (us, this kernel and the best other tile): int8, 768 to 1,152 columns, 17,920 rows (11 blocks)
-// 25.3 and 25.2, 35,000 40.7 and 44.3, 69,930 75.1 and 92.2; 768 to 2 x 992 gated, 7,000 (7) 19.8 and 17.2, 17,920 (17)
-// 35.5 and 38.3, 69,930 113 and 141; 256 to 2 x 1,024 gated, 17,920 (9) 21.5 and 20.0, 69,930 (34) 56.4 and 64.2; 256 to 832,
+// 26.0 and 26.8, 35,000 40.1 and 44.4, 69,930 69.3 and 87.3; 768 to 2 x 992 gated, 7,000 (7) 19.8 and 17.2, 17,920 (17) 35.5
+// and 38.3, 69,930 113 and 141; 256 to 2 x 1,024 gated, 17,920 (9) 21.5 and 20.0, 69,930 (34) 56.4 and 64.2; 256 to 832,
 // 17,920 (4) 14.9 and 11.7, 69,930 (17) 31.6 and 35.4; 1,024 to 768 with the residual and the mix, 17,920 (7) 29.4 and 32.2,
 // 35,000 (13) 46.8 and 54.4; 1,024 to 256 so, 35,000 (4) 25.7 and 25.0, 69,930 (9) 36.5 and 41.1; fp16, 256 to 256 with bias
-// and residual, 69,930 (9) 22.4 and 24.5. (Left out, as no faster: the residual at depths 512 and 768.) A launch of one output a
-// weight row that writes more than the last-level cache holds is bound by its writes, and whole lines from LDS go faster than
-// these 16-byte stores (512 to 2,048 at 65,536 rows, 268 MB: 121 us and 109 on tile 4); gated, 293 MB still take 163 and 240. For
-// output rows of whole KB, whose 32 rows a store falls on few of L2's channels, from short inputs and without a residual to
-// read that is so from 230 MiB on (this kernel and tile 4: 512 to 1,024, 210 MiB 90 and 92, 230 MiB 116 and 100; 512 to 1,536, 220
-// MiB 95 and 95, 240 MiB 115 and 100; 512 to 2,048, 230 MiB 99 and 100, 255 MiB 120 and 110; 256 to 2,048, 240 MiB 73 and 76, 250
-// MiB 84 and 77), for others not up to 256 MiB (512 to 1,600, 230 MiB 80 and 103, 255 MiB 106 and 116; 768 to 1,152, 255 MiB 139
-// and 150; 1,024 to 1,024 with the residual 163 and 239; fp16, 512 to 512 144 and 195).
-// Below LARGE_ROWS, where the other tile is 11 and not the slower 4, a plan whose workgroups are too often out of work does not
-// pay: 768 to 2 x 2,176 (17 groups for 32 workgroups, busy 0.53) at 12,000 rows 68.5 and 59.9, 256 to 2 x 4,352 65.9 and 49.1 (at
-// 35,000 177 and 174, at 70,000 345 and 333; 512 to 2 x 4,352 208 and 241), 512 to 2 x 2,816 (11 groups, 0.69) 49.8 and 52.5; with the
-// shorter MFMA chains of depth 256 the line lies higher, 256 to 2 x 2,816 39.6 and 34.1. Two working wavefronts of a sole group's
-// eight do not either: 256 to 72 at 110,000 rows 18.4 and 14.1, 512 to 72 19.8 and 19.0 (three, 768 to 72: 20.9 and 23.4). Beside a
+// and residual, 69,930 (9) 22.4 and 24.5. (Left out, as no faster: the residual at depths 512 and 768.) A launch of one
+// output a weight row that writes more than the last-level cache holds is bound by its writes, and whole lines from LDS go
+// faster than these 16-byte stores (512 to 2,048 at 65,536 rows, 268 MB: 121 us and 109 on tile 4); gated, 293 MB still take
+// 163 and 240. For output rows of whole KB, from short inputs and without a residual to read, that is so from 230 MiB on
+// (this kernel and tile 4: 512 to 1,024, 210 MiB 90 and 92, 230 MiB 116 and 100; 512 to 1,536, 220 MiB 95 and 95, 240 MiB 115
+// and 100; 512 to 2,048, 230 MiB 99 and 100, 255 MiB 120 and 110; 256 to 2,048, 240 MiB 73 and 76, 250 MiB 84 and 77), for
+// others not up to 256 MiB (512 to 1,600, 230 MiB 80 and 103, 255 MiB 106 and 116; 768 to 1,152, 255 MiB 139 and 150; 1,024
+// to 1,024 with the residual 163 and 239; fp16, 512 to 512 144 and 195). Below LARGE_ROWS, where the other tile is 11 and not
+// the slower 4, a plan whose workgroups are too often out of work does not pay: 768 to 2 x 2,176 (17 groups for 32
+// workgroups, busy 0.53) at 12,000 rows 68.5 and 59.9, 256 to 2 x 4,352 65.9 and 49.1 (at 35,000 177 and 174, at 70,000 345
+// and 333; 512 to 2 x 4,352 208 and 241), 512 to 2 x 2,816 (11 groups, 0.69) 49.8 and 52.5; with the shorter MFMA chains of
+// depth 256 the line lies higher, 256 to 2 x 2,816 39.6 and 34.1. Two working wavefronts of a sole group's eight do not
+// either: 256 to 72 at 110,000 rows 18.4 and 14.1, 512 to 72 19.8 and 19.0 (three, 768 to 72: 20.9 and 23.4). Beside a
 // residual a part-filled group costs a full one, which near the line is no loss yet: 1,024 to 264 and 384 at 25,000 rows 22.9
 // and 24.1, where tile 13 takes 23.9 and 24.3; with the mix 27.0 and 29.2, and 26.9 and 27.9.
 constexpr int STREAM_BLOCKS = 10, DEEP_STREAM_BLOCKS = 6, F16_STREAM_BLOCKS = 8, LARGE_ROWS = 32768;

@@ -37,8 +37,9 @@ LINEAR_TILES = {"gfx950": [(5, 1), (9, 3), (48, 6), (100, 11), (math.inf, 15)]}
 RESIDENT_TILE, RESIDENT_DEPTH = 15, 512
 RESIDENT_OUTPUT_BYTES, RESIDENT_COLUMNS = 1 << 31, 32 * 256   # its outputs' (32-bit offsets) and its column groups' limits
 # and from this share on where it has 1,024 columns or more, so that each of its workgroups still has a long stream of row
-# blocks (512 to 1,600 columns at 17,920 rows, graphs of launches: 37.4 against 43.0 us on tile 11); up to 4,096, inside the
-# column groups and output bytes it takes
+# blocks (graphs of launches, tile 15 and 11, us: 512 to 1,600 columns at 17,920 rows 40.1 and 46.6, at 12,800 30.6 and 35.6; to
+# 1,280 at 12,544 rows 27.6 and 26.8, at 13,312 27.8 and 29.8; to 1,024 at 12,544 24.7 and 26.5, at 16,384 27.4 and 26.1, with the
+# residual 28.3 and 31.3), up to the 4,096 it was timed with (12,800 rows 58.3 and 77.6)
 RESIDENT_WIDE_SHARE, RESIDENT_WIDE_COLUMNS = 48, range(1024, 4097)
 # gated, rows of whole lines (tile 12 stages 128 bytes of a row) from 1 KB on; others keep LINEAR_TILES. Graphs of launches, us:
 # 512 to 2 x 2,048 4,480 rows 27.5 on tile 12 and 29.3 on tile 6, 1,024 to 2 x 2,816 63.3 and 69.7, but 256 to 2 x 1,024 12.1 and

@@ -56,9 +56,12 @@ INT8_DEPTH = 64
 INT8_TILES = {"gfx950": {"projection": [(0.55, 14), (5, 1), (9, 8), (100, 11), (math.inf, 15)],
                          "gate_up": [(0.3, 14), (4, 1), (18, 9), (40, 10), (math.inf, 15)],
                          "down": [(0.55, 14), (8, 1), (32, 6), (48, 5), (math.inf, 16)]}}
-# projection of rows longer than 512 (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 7.9 us on tile 6 and
-# 9.0 on tile 11, 7,000 in 11.3 on tile 13 and 12.7, 17,920 in 25.2 and 27.8; past them tile 0, which takes the weights in
-# registers at such depths too (35,000 rows: 40.7 against 47.1 us on tile 13, 69,930 75.1 against 98.2)
+# projection of rows longer than 512 (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 8.1 us on tile 6 and
+# 9.1 on tile 11, 7,000 in 12.1 on tile 13 and 13.8, 17,920 in 26.8 and 29.5; past them tile 0, which takes the weights in
+# registers at such depths too (35,000 rows: 40.1 against 44.4 us on tile 4, 69,930 69.3 against 87.3). At other depths and
+# columns (768 to 768 and 2,400, 1,024 to 1,152 and 1,600, 1,536 to 1,536, 2,048 to 1,024; 17 counts of rows each) the lines
+# gain up to 18% on tile 11 and lose at most 6%, where a last wave of workgroups falls badly (1,024 to 1,600 at 5,100 rows 18.3 and
+# 17.4, 768 to 768 at 13,000 17.4 and 16.4).
 # (for the shipped table only: one put in INT8_TILES in its place, or edited there, holds for every depth)
 LONG_PROJECTION_TILES = {"gfx950": [(0.55, 14), (5, 1), (9, 8), (20, 6), (75, 13), (math.inf, 0)]}
 SHIPPED_PROJECTION_TILES = list(INT8_TILES["gfx950"]["projection"])
