@@ -504,12 +504,19 @@ void template_attention_wave_kernel(
     }
 }
 
-// The launch's mode by its pairs: FOURS while each of its places (a workgroup of four wavefronts: two a SIMD for 64 wide
-// heads' 175 registers, four for the narrow ones' 121) takes one or two, past them WHOLE. Timed both ways on an MI355X (us,
-// FOURS and WHOLE), 70 tokens: 8 x 64 heads, batch 96 14.2 and 17.7, 128 (1,024 pairs, two a place) 18.0 and 18.8, 192 25.4 and
-// 19.6; 12 groups of 16 and 32 wide, batch 84 18.4 and 27.1, 128 (1,536 pairs) 23.6 and 29.3, 200 35.8 and 31.1; 8 x 32 heads,
-// batch 192 (1,536 pairs) 16.6 and 18.3, 300 25.6 and 20.3. Over the 64 squares alone WHOLE's waves have no fifth slab: 8 x 64
-// heads, batch 100 (800 pairs) 16.1 and 14.0.
+// The launch's mode by n, its pairs a compute unit (rounded up). FOURS's workgroups of four wavefronts, one a SIMD each,
+// take a time that grows with n; WHOLE's wavefronts, one or two (narrow widths: up to three) a SIMD, much the same for n of
+// 1 to 4 and of 5 to 8, and longer the more heads a pair has. So a head a pair takes WHOLE from n = 3 (4 where the values
+// are wider than the queries), several heads from 4, but three or more not at 5, nor, of narrow widths over five tiles, two
+// or more up to 6. Timed both ways on an MI355X (us, FOURS and WHOLE, at 512, 768, 1,024, 1,280 and 1,536 pairs): 8 x 64
+// heads over 64 tokens 9.3 and 9.9, 12.4 and 11.1, 16.6 and 12.0, 18.4 and 14.7, 22.5 and 15.8, over 70 10.8 and 12.1, 14.2
+// and 13.2, 18.0 and 14.2, 20.3 and 18.6, 25.0 and 19.7; 16 on 4 x 32 over 64 tokens 13.4 and 20.1, 17.8 and 21.6, 22.4 and
+// 22.2, 26.1 and 29.1, 30.2 and 29.8, over 70 17.3 and 25.5, 21.8 and 26.9, 27.0 and 28.1, 31.6 and 37.4, 36.0 and 37.9; 24
+// on 12, query width 16, value width 32, over 70 11.3 and 14.7, 14.3 and 15.6, 18.1 and 16.2, 19.7 and 22.2, 22.4 and 23.0;
+// past 1,536 pairs WHOLE wins everywhere. Its workgroups, one a compute unit, share the pairs out evenly however few they
+// are: filled with a pair for each wavefront instead, 1,024 pairs of 16 on 4 x 32 heads over 64 tokens had 86 workgroups
+// and took 36.0 us, where the kernel before this one took 23.9 (70 tokens, 8 x 64 heads, 1,032 pairs: 18.5 against 16.6
+// now).
 template <int DQP, int DV, int TILES, bool BF16>
 int launch_waves(const void* projected, const void* keyed, const void* q_gain, const void* k_gain, void* out, int B, int T, int heads,
                  int kv_heads, int dq, int templates_count, float eps, float scale, hipStream_t stream)
@@ -526,10 +533,10 @@ int launch_waves(const void* projected, const void* keyed, const void* q_gain, c
         return launch_status();
     };
     typedef WaveLayout<DQP, DV, TILES, WHOLE> L;
-    const int most = (L::NARROW ? 6 : 4) * units / (TILES == 4 ? 2 : 1);
-    if (pairs > most)
-        return launch(std::integral_constant<AttentionMode, WHOLE>{}, min(units, (pairs + L::WAVES - 1) / L::WAVES));
-    return launch(std::integral_constant<AttentionMode, FOURS>{}, min((L::NARROW ? 4 : 2) * units, pairs));
+    const int n = (pairs + units - 1) / units;
+    const bool fours = heads == kv_heads ? n <= (DV > DQP ? 3 : 2) : L::NARROW && TILES == 5 ? n <= 6 : n <= 3 || (n == 5 && heads > 2 * kv_heads);
+    if (fours) return launch(std::integral_constant<AttentionMode, FOURS>{}, min((L::NARROW ? 4 : 2) * units, pairs));
+    return launch(std::integral_constant<AttentionMode, WHOLE>{}, min(units, pairs));
 }
 
 }  // namespace

@@ -720,10 +720,11 @@ def test_groups_a_workgroup_change_no_bit(device, heads, kv_heads, dq, dv, token
         launch_template_attention(*arguments, groups_per_block=5)   # not a divisor of the pairs
 
 
-def whole_pair_positions(device, kv_heads, dq, dv):
-    """A few positions more than the most that the kernel of widths up to 64 shares over four wavefronts a pair (65 to 80 tokens)."""
+def whole_pair_positions(device, kv_heads):
+    """A few positions more than the most that the kernel of widths up to 64 shares over four wavefronts a pair: six pairs a compute
+    unit, of several narrow heads each, over 65 to 80 tokens."""
     units = torch.cuda.get_device_properties(device).multi_processor_count
-    return (6 if dq <= 32 and dv <= 32 else 4) * units // kv_heads + 5
+    return 6 * units // kv_heads + 5
 
 
 @pytest.mark.parametrize("heads, kv_heads, dq, dv, tokens", [(8, 8, 64, 64, 70), (8, 4, 32, 32, 80), (4, 4, 16, 64, 65), (6, 3, 64, 16, 66)])
@@ -732,7 +733,7 @@ def test_large_attention_launches_give_the_small_launchs_bits(device, heads, kv_
     same bits as in launches of seven positions (four wavefronts a pair), and the answer is the fp32 formula's. The grouped case
     with two heads a group (6 on 3) once differed on the tokens past the squares of a few positions in the middle of the
     launch."""
-    positions = whole_pair_positions(device, kv_heads, dq, dv)
+    positions = whole_pair_positions(device, kv_heads)
     arguments = attention_operands(device, positions, heads, kv_heads, dq, dv, seed=tokens, tokens=tokens)
     large = template_attention(*arguments)
     assert torch.allclose(large.float(), reference_attention(arguments), atol=1e-2)
@@ -742,18 +743,19 @@ def test_large_attention_launches_give_the_small_launchs_bits(device, heads, kv_
 
 @pytest.mark.parametrize("heads, kv_heads, dq, dv, tokens, count, positions", [
     (8, 8, 64, 64, 70, 8, 129), (8, 8, 64, 64, 64, 8, 65), (4, 4, 40, 64, 66, 6, 257), (24, 12, 24, 32, 70, 8, 129), (8, 4, 8, 16, 80, 3, 385),
-    (2, 1, 32, 32, 65, 8, 1537)])
+    (2, 1, 32, 32, 65, 8, 1537), (8, 4, 32, 32, 64, 8, 193), (12, 4, 32, 32, 64, 8, 257), (4, 4, 32, 64, 70, 8, 193)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_both_sharings_of_the_pairs_give_the_same_bits(device, heads, kv_heads, dq, dv, tokens, count, positions, dtype):
-    """Widths up to 64 and up to 80 tokens: a launch just past four pairs a compute unit (two over 64 tokens; six of widths up
-    to 32) gives its wavefronts whole pairs, and one of a few positions shares a pair over four. The same bits, the fp32
-    formula's answer, at the smallest and largest token counts, query widths that do not fill their chunks and fewer than
+    """Widths up to 64 and up to 80 tokens: a launch of some pairs a compute unit (more than two of one head each; four, or seven of
+    narrow widths over 65 tokens and more, of several; not five of three: the last shape but one) gives its wavefronts whole pairs, and one
+    of a few positions shares a pair over four. The same bits, the fp32 formula's answer, at the smallest and largest token counts, query widths that do not fill their chunks and fewer than
     eight templates; a position of infinities and NaNs stays its own."""
     projected, *rest = attention_operands(device, positions, heads, kv_heads, dq, dv, seed=tokens + dq, tokens=tokens, templates_count=count)
     projected = projected.to(dtype)
     arguments = (projected, *rest)
-    whole = template_attention(*arguments)
-    assert (whole.float() - reference_attention(arguments)).abs().max() < 1e-2
+    whole, expected = template_attention(*arguments), reference_attention(arguments)
+    # 1e-2, and for bf16 outputs their own rounding, up to half a step of 8 bits: 2^-9 of the value (outputs reach 4 here)
+    assert ((whole.float() - expected).abs() <= 1e-2 + (2 ** -9 * expected.abs() if dtype == torch.bfloat16 else 0)).all()
     some = [0, 1, 2, positions // 2, positions - 2, positions - 1]
     assert torch.equal(template_attention(projected[some].contiguous(), *arguments[1:]), whole[some])
     spoilt = projected.clone()
@@ -829,7 +831,7 @@ def test_bf16_template_attention_at_64_tokens_with_a_bias_per_head(device, posit
 
 def test_large_bf16_attention_launches_give_the_small_launchs_bits(device):
     """bf16 rows at 70 tokens, a wavefront a pair: a position's rows are a three-position launch's bits."""
-    positions = whole_pair_positions(device, 8, 64, 64)
+    positions = whole_pair_positions(device, 8)
     arguments = bf16_operands(attention_operands(device, positions, 8, 8, 64, 64, seed=70, tokens=70))
     large = template_attention(*arguments)
     assert (large.float() - reference_attention(arguments)).abs().max() < 1e-2
