@@ -56,13 +56,15 @@ INT8_DEPTH = 64
 INT8_TILES = {"gfx950": {"projection": [(0.55, 14), (5, 1), (9, 8), (100, 11), (math.inf, 15)],
                          "gate_up": [(0.3, 14), (4, 1), (18, 9), (40, 10), (math.inf, 15)],
                          "down": [(0.55, 14), (8, 1), (32, 6), (48, 5), (math.inf, 16)]}}
-# projection of rows longer than 512 (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 8.1 us on tile 6 and
+# projection of rows of 768 or more (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 8.1 us on tile 6 and
 # 9.1 on tile 11, 7,000 in 12.1 on tile 13 and 13.8, 17,920 in 26.8 and 29.5; past them tile 0, which takes the weights in
 # registers at such depths too (35,000 rows: 40.1 against 44.4 us on tile 4, 69,930 69.3 against 87.3). At other depths and
 # columns (768 to 768 and 2,400, 1,024 to 1,152 and 1,600, 1,536 to 1,536, 2,048 to 1,024; 17 counts of rows each) the lines
 # gain up to 18% on tile 11 and lose at most 6%, where a last wave of workgroups falls badly (1,024 to 1,600 at 5,100 rows 18.3 and
-# 17.4, 768 to 768 at 13,000 17.4 and 16.4).
+# 17.4, 768 to 768 at 13,000 17.4 and 16.4). Rows of 640 keep the table (to 640, 960, 1,280 and 1,600 columns tile 13 takes up to 11%
+# more than tile 11: 640 to 1,280 at 8,785 rows 16.4 and 15.5, 640 to 640 at 14,000 15.8 and 14.2).
 # (for the shipped table only: one put in INT8_TILES in its place, or edited there, holds for every depth)
+LONG_PROJECTION_DEPTH = 768
 LONG_PROJECTION_TILES = {"gfx950": [(0.55, 14), (5, 1), (9, 8), (20, 6), (75, 13), (math.inf, 0)]}
 SHIPPED_PROJECTION_TILES = list(INT8_TILES["gfx950"]["projection"])
 # the split-K tile's wavefronts: each reads 1, 2 or 4 steps of 128 bytes of K, and the outputs go 8 columns a lane
@@ -148,7 +150,7 @@ def int8_tile(device: torch.device, matmul: str, M: int, N: int = 0, K: int = 0,
     takes them: 0, the kernel's own pick of a whole-K tile, which takes every shape)."""
     arch, units = hip_kernels.gpu(device)
     tiles = INT8_TILES.get(arch, INT8_TILES["gfx950"])[matmul]
-    if matmul == "projection" and tiles == SHIPPED_PROJECTION_TILES and K > RESIDENT_DEPTH and K % 128 == 0:
+    if matmul == "projection" and tiles == SHIPPED_PROJECTION_TILES and K >= LONG_PROJECTION_DEPTH and K % 128 == 0:
         tiles = LONG_PROJECTION_TILES.get(arch, LONG_PROJECTION_TILES["gfx950"])
     share = M / units
     candidates = [tile for most, tile in tiles if share <= most]

@@ -21,7 +21,7 @@ def test_tile_for_takes_the_first_row_share_that_fits():
 def test_a_projection_table_put_in_the_shipped_ones_place_holds_at_every_depth(monkeypatch):
     monkeypatch.setattr(hip_kernels, "gpu", lambda device: ("gfx950", 256))
     chosen = lambda K: int8_blocks.int8_tile(torch.device("cuda"), "projection", 3570, 1152, K, bias=True)
-    assert (chosen(512), chosen(768), chosen(832)) == (11, 6, 11)   # 832: no whole 128-byte lines
+    assert (chosen(512), chosen(640), chosen(768), chosen(832)) == (11, 11, 6, 11)   # 832: no whole 128-byte lines
     monkeypatch.setitem(int8_blocks.INT8_TILES["gfx950"], "projection", [(math.inf, 3)])
     assert (chosen(512), chosen(768)) == (3, 3)
     monkeypatch.setitem(int8_blocks.INT8_TILES["gfx950"], "projection", list(int8_blocks.SHIPPED_PROJECTION_TILES))   # put back
