@@ -58,13 +58,15 @@ INT8_TILES = {"gfx950": {"projection": [(0.55, 14), (5, 1), (9, 8), (100, 11), (
                          "down": [(0.55, 14), (8, 1), (32, 6), (48, 5), (math.inf, 16)]}}
 # projection of rows of 768 or more (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 8.1 us on tile 6 and
 # 9.1 on tile 11, 7,000 in 12.1 on tile 13 and 13.8, 17,920 in 26.8 and 29.5; past them tile 0, which takes the weights in
-# registers at such depths too (35,000 rows: 40.1 against 44.4 us on tile 4, 69,930 69.3 against 87.3). At other depths and
-# columns (768 to 768 and 2,400, 1,024 to 1,152 and 1,600, 1,536 to 1,536, 2,048 to 1,024; 17 counts of rows each) the lines
-# gain up to 18% on tile 11 and lose at most 6%, where a last wave of workgroups falls badly (1,024 to 1,600 at 5,100 rows 18.3 and
-# 17.4, 768 to 768 at 13,000 17.4 and 16.4). Rows of 640 keep the table (to 640, 960, 1,280 and 1,600 columns tile 13 takes up to 11%
+# registers at such depths too (35,000 rows: 40.1 against 44.4 us on tile 4, 69,930 69.3 against 87.3). Where the
+# last round of workgroups would be small, tile 11 (long_projection_tile): past 256 of tile 6's (768 to 1,152 at 3,570 rows, 252 of
+# them, 8.1 against 9.1 us on tile 11, at 3,873, 279, 10.5 and 9.6; 1,024 to 1,600 at 5,100 18.3 and 17.4), and where tile 13's last
+# 512 places are less than LEAST_LAST_ROUND full (768 to 960 at 8,785, 552, 16.9 and 14.9; 768 to 768 at 13,000, 612, 17.4 and 16.4;
+# 1,024 to 1,600 at 7,000, 715, 20.5 and 19.6; but 768 to 960 at 12,000, 752, 17.7 and 18.2).
+# Rows of 640 keep the table (to 640, 960, 1,280 and 1,600 columns tile 13 takes up to 11%
 # more than tile 11: 640 to 1,280 at 8,785 rows 16.4 and 15.5, 640 to 640 at 14,000 15.8 and 14.2).
 # (for the shipped table only: one put in INT8_TILES in its place, or edited there, holds for every depth)
-LONG_PROJECTION_DEPTH = 768
+LONG_PROJECTION_DEPTH, LEAST_LAST_ROUND = 768, 0.43
 LONG_PROJECTION_TILES = {"gfx950": [(0.55, 14), (5, 1), (9, 8), (20, 6), (75, 13), (math.inf, 0)]}
 SHIPPED_PROJECTION_TILES = list(INT8_TILES["gfx950"]["projection"])
 # the split-K tile's wavefronts: each reads 1, 2 or 4 steps of 128 bytes of K, and the outputs go 8 columns a lane
@@ -142,6 +144,17 @@ def tile_takes(tile: int, N: int, K: int, gated: bool = False, bias: bool = Fals
     return waves is None or (N % 8 == 0 and K % (128 * waves) == 0 and K // (128 * waves) in (1, 2, 4))
 
 
+def long_projection_tile(tile: int, M: int, N: int, units: int) -> int:
+    """LONG_PROJECTION_TILES' tile, or 11 where the last round of its workgroups is too small: tile 6 holds one of 128 x 128 a compute
+    unit and pays in its first round alone, tile 13 two, and pays where the last round fills LEAST_LAST_ROUND of them."""
+    workgroups = -(-M // 128) * -(-N // 128)
+    if tile == 6:
+        return tile if workgroups <= units else 11
+    if tile == 13:
+        return tile if (workgroups - 1) % (2 * units) + 1 >= LEAST_LAST_ROUND * 2 * units else 11
+    return tile
+
+
 def int8_tile(device: torch.device, matmul: str, M: int, N: int = 0, K: int = 0, gated: bool | None = None, bias: bool = False,
               residual: bool | None = None) -> int:
     """The tile of int8_linear for M rows of matmul (reference int8_blocks.py:39-42, keyed by gfx target, not capability):
@@ -152,6 +165,7 @@ def int8_tile(device: torch.device, matmul: str, M: int, N: int = 0, K: int = 0,
     tiles = INT8_TILES.get(arch, INT8_TILES["gfx950"])[matmul]
     if matmul == "projection" and tiles == SHIPPED_PROJECTION_TILES and K >= LONG_PROJECTION_DEPTH and K % 128 == 0:
         tiles = LONG_PROJECTION_TILES.get(arch, LONG_PROJECTION_TILES["gfx950"])
+        tiles = [(most, long_projection_tile(tile, M, N, units) if N else tile) for most, tile in tiles]
     share = M / units
     candidates = [tile for most, tile in tiles if share <= most]
     gated = matmul == "gate_up" if gated is None else gated

@@ -58,7 +58,17 @@ def test_no_choice_of_an_int8_block_asks_torch_for_its_properties(monkeypatch):
             fused_blocks.linear_tile(device, M, f32, 1024, gated, 512)
 
 
+@pytest.mark.parametrize("M, N, expected", [(3584, 1152, 6), (3585, 1152, 11), (7000, 1152, 13), (8785, 960, 11), (12000, 960, 13),
+                                            (13000, 768, 11), (17920, 1152, 13), (19200, 1152, 13), (19201, 1152, 0)])
+def test_long_projections_leave_tiles_whose_last_round_is_small(monkeypatch, M, N, expected):
+    monkeypatch.setattr(hip_kernels, "gpu", lambda device: ("gfx950", 256))
+    assert int8_blocks.int8_tile(torch.device("cuda"), "projection", M, N, 768, bias=True) == expected
+
+
 @pytest.mark.parametrize("M, K, N, gated, f32, bias, expected", [
+    (8192, 768, 768, False, False, True, 12), (8193, 768, 768, False, False, True, 13), (10880, 768, 768, False, False, True, 13),
+    (10881, 768, 768, False, False, True, 12), (8193, 768, 768, False, True, True, 13), (6453, 768, 1152, False, False, True, 13),
+    (8193, 512, 768, False, True, True, 12),
     (256 * 48, 512, 1600, False, False, True, 6), (256 * 48 + 1, 512, 1600, False, False, True, 15),    # the long streams' first row
     (256 * 49, 512, 1016, False, False, True, 11), (256 * 49, 512, 1024, False, False, True, 15),        # and least columns
     (256 * 49, 512, 1604, False, False, True, 11), (256 * 49, 512, 1600, False, False, False, 11),       # no whole 8 columns; no bias
