@@ -72,11 +72,12 @@ LONG_ROW_BYTES, MANY_TILES_ROW_BYTES, SMALL_TILES_A_UNIT = 1536, 2048, 1.6
 # (csrc/attention_wave.h) and take any run of pairs a workgroup; the others take groups_per_workgroup's
 ATTENTION_SHARING_TOKENS, ATTENTION_SHARING_WIDTH = 80, 64
 
-# Where tile 12's 128 x 64 workgroups are more than the compute units hold at once (three each: 48 KB of LDS) and 128 x 128 ones are
-# not (two each), rows of ONE_ROUND_ROW_BYTES or more that a table gives to 12 take 13: one round of workgroups, not one and a remainder (768 inputs:
-# to 768 at 9,000 rows 852 and 426 of them, 21.7 and 17.1 us, to 1,152 at 6,453 22.3 and 17.3, f32 out to 768 at 9,000 27.3 and 23.1;
-# but to 768 at 8,000, 756, 15.6 and 16.5, and at 11,000, 1,032 and 516, 23.5 and 26.2. Of 768 to 2,048 inputs everywhere between the
-# two, by 1.17 to 1.36; f32 out of 640 to 1,024 by 0.95 to 1.26, of 512 by 0.93 to 1.12, of 256 by 0.80 to 1.04)
+# Where tile 12's 128 x 64 workgroups are more than the compute units hold at once (three each: 48 KB of LDS) and 128 x 128
+# ones are not (two each), rows of ONE_ROUND_ROW_BYTES or more that a table gives to 12 take 13: one round of workgroups,
+# not one and a remainder (768 inputs: to 768 at 9,000 rows 852 and 426 of them, 21.7 and 17.1 us, to 1,152 at 6,453 22.3
+# and 17.3, f32 out to 768 at 9,000 27.3 and 23.1; but to 768 at 8,000, 756, 15.6 and 16.5, and at 11,000, 1,032 and 516,
+# 23.5 and 26.2. Of 768 to 2,048 inputs everywhere between the two, by 1.17 to 1.36; f32 out of 640 to 1,024 by 0.95 to
+# 1.26, of 512 by 0.93 to 1.12, of 256 by 0.80 to 1.04)
 ONE_ROUND, ONE_ROUND_ROW_BYTES = {12: (128, 64, 3), 13: (128, 128, 2)}, 1280   # each tile's (rows, columns, workgroups a compute unit)
 
 

@@ -56,16 +56,16 @@ INT8_DEPTH = 64
 INT8_TILES = {"gfx950": {"projection": [(0.55, 14), (5, 1), (9, 8), (100, 11), (math.inf, 15)],
                          "gate_up": [(0.3, 14), (4, 1), (18, 9), (40, 10), (math.inf, 15)],
                          "down": [(0.55, 14), (8, 1), (32, 6), (48, 5), (math.inf, 16)]}}
-# projection of rows of 768 or more (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 8.1 us on tile 6 and
-# 9.1 on tile 11, 7,000 in 12.1 on tile 13 and 13.8, 17,920 in 26.8 and 29.5; past them tile 0, which takes the weights in
-# registers at such depths too (35,000 rows: 40.1 against 44.4 us on tile 4, 69,930 69.3 against 87.3). Where the
-# last round of workgroups would be small, tile 11 (long_projection_tile): past 256 of tile 6's (768 to 1,152 at 3,570 rows, 252 of
-# them, 8.1 against 9.1 us on tile 11, at 3,873, 279, 10.5 and 9.6; 1,024 to 1,600 at 5,100 18.3 and 17.4), and where tile 13's last
-# 512 places are less than LEAST_LAST_ROUND full (768 to 960 at 8,785, 552, 16.9 and 14.9; 768 to 768 at 13,000, 612, 17.4 and 16.4;
-# 1,024 to 1,600 at 7,000, 715, 20.5 and 19.6; but 768 to 960 at 12,000, 752, 17.7 and 18.2).
-# Rows of 640 keep the table (to 640, 960, 1,280 and 1,600 columns tile 13 takes up to 11%
-# more than tile 11: 640 to 1,280 at 8,785 rows 16.4 and 15.5, 640 to 640 at 14,000 15.8 and 14.2).
-# (for the shipped table only: one put in INT8_TILES in its place, or edited there, holds for every depth)
+# projection of rows of 768 or more (768 to 1,152 columns, graphs of launches on an MI355X): 3,570 rows in 8.1 us on tile 6
+# and 9.1 on tile 11, 7,000 in 12.1 on tile 13 and 13.8, 17,920 in 26.8 and 29.5; past them tile 0, which takes the weights
+# in registers at such depths too (35,000 rows: 40.1 against 44.4 us on tile 4, 69,930 69.3 against 87.3). Where the last
+# round of workgroups would be small, tile 11 (long_projection_tile): past 256 of tile 6's (768 to 1,152 at 3,570 rows, 252
+# of them, 8.1 against 9.1 us on tile 11, at 3,873, 279, 10.5 and 9.6; 1,024 to 1,600 at 5,100 18.3 and 17.4), and where
+# tile 13's last 512 places are less than LEAST_LAST_ROUND full (768 to 960 at 8,785, 552, 16.9 and 14.9; 768 to 768 at
+# 13,000, 612, 17.4 and 16.4; 1,024 to 1,600 at 7,000, 715, 20.5 and 19.6; but 768 to 960 at 12,000, 752, 17.7 and 18.2).
+# Rows of 640 keep the table (to 640, 960, 1,280 and 1,600 columns tile 13 takes up to 11% more than tile 11: 640 to 1,280
+# at 8,785 rows 16.4 and 15.5, 640 to 640 at 14,000 15.8 and 14.2). (for the shipped table only: one put in INT8_TILES in
+# its place, or edited there, holds for every depth)
 LONG_PROJECTION_DEPTH, LEAST_LAST_ROUND = 768, 0.43
 LONG_PROJECTION_TILES = {"gfx950": [(0.55, 14), (5, 1), (9, 8), (20, 6), (75, 13), (math.inf, 0)]}
 SHIPPED_PROJECTION_TILES = list(INT8_TILES["gfx950"]["projection"])
