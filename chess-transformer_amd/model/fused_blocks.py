@@ -77,13 +77,15 @@ ATTENTION_SHARING_TOKENS, ATTENTION_SHARING_WIDTH = 80, 64
 # not one and a remainder (768 inputs: to 768 at 9,000 rows 852 and 426 of them, 21.7 and 17.1 us, to 1,152 at 6,453 22.3
 # and 17.3, f32 out to 768 at 9,000 27.3 and 23.1; but to 768 at 8,000, 756, 15.6 and 16.5, and at 11,000, 1,032 and 516,
 # 23.5 and 26.2. Of 768 to 2,048 inputs everywhere between the two, by 1.17 to 1.36; f32 out of 640 to 1,024 by 0.95 to
-# 1.26, of 512 by 0.93 to 1.12, of 256 by 0.80 to 1.04)
+# 1.26; of 512 by 1.01 to 1.12 up to half a workgroup more a compute unit, 512 to 512 at 12,900 rows 20.4 and 18.4, and 0.93
+# to 0.97 past it; of 256 by 0.80 to 1.04)
 ONE_ROUND, ONE_ROUND_ROW_BYTES = {12: (128, 64, 3), 13: (128, 128, 2)}, 1280   # each tile's (rows, columns, workgroups a compute unit)
+SMALL_REMAINDER_ROW_BYTES, SMALL_REMAINDER = 1024, 0.5
 
 
-def in_one_round(tile: int, M: int, N: int, units: int) -> bool:
+def in_one_round(tile: int, M: int, N: int, units: int, more: float = 0) -> bool:
     rows, columns, held = ONE_ROUND[tile]
-    return -(-M // rows) * -(-N // columns) <= held * units
+    return -(-M // rows) * -(-N // columns) <= (held + more) * units
 
 
 # tiles lists (share, tile) pairs by growing share; a launch takes the first whose share bounds M / multiprocessors (the last bounds any)
@@ -113,8 +115,9 @@ def linear_tile(device: torch.device, M: int, accumulate_fp32: bool = False, row
     else:
         table = LINEAR_TILES
     tile = tile_for(table.get(arch, table["gfx950"]), M, units)
-    if tile == 12 and row_bytes >= ONE_ROUND_ROW_BYTES and not gated and N and not in_one_round(12, M, N, units) and in_one_round(13, M, N, units):
-        return 13
+    if tile == 12 and not gated and N and not in_one_round(12, M, N, units) and in_one_round(13, M, N, units):
+        small = row_bytes >= SMALL_REMAINDER_ROW_BYTES and in_one_round(12, M, N, units, SMALL_REMAINDER)
+        return 13 if small or row_bytes >= ONE_ROUND_ROW_BYTES else 12
     return tile
 
 

@@ -68,7 +68,8 @@ def test_long_projections_leave_tiles_whose_last_round_is_small(monkeypatch, M, 
 @pytest.mark.parametrize("M, K, N, gated, f32, bias, expected", [
     (8192, 768, 768, False, False, True, 12), (8193, 768, 768, False, False, True, 13), (10880, 768, 768, False, False, True, 13),
     (10881, 768, 768, False, False, True, 12), (8193, 768, 768, False, True, True, 13), (6453, 768, 1152, False, False, True, 13),
-    (8193, 512, 768, False, True, True, 12),
+    (8193, 512, 768, False, True, True, 13), (9472, 512, 768, False, True, True, 13), (9473, 512, 768, False, True, True, 12),
+    (8193, 256, 768, False, True, True, 12),
     (256 * 48, 512, 1600, False, False, True, 6), (256 * 48 + 1, 512, 1600, False, False, True, 15),    # the long streams' first row
     (256 * 49, 512, 1016, False, False, True, 11), (256 * 49, 512, 1024, False, False, True, 15),        # and least columns
     (256 * 49, 512, 1604, False, False, True, 11), (256 * 49, 512, 1600, False, False, False, 11),       # no whole 8 columns; no bias
